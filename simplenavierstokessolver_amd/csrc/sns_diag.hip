@@ -154,14 +154,41 @@ __global__ void __launch_bounds__(kDiagThreads)
 }
 
 // Reduces nb partial slots and applies the normalisations of
-// src/logging.c:201,219-220,247-248,266.
-__global__ void __launch_bounds__(64)
+// src/logging.c:201,219-220,247-248,266.  One workgroup of 64 threads per
+// slot kind: a thread's entries k*kFinalThreads + t all belong to slot kind
+// t % kDiagSlots, so the loads are contiguous across the workgroup and
+// kFinalUnroll of them are in flight per thread; the 64 sums of a slot kind
+// are then added in a fixed order.  Latency bounds it (at most 2048 x 11
+// values): one thread per slot kind adding them one after another took 303
+// us for 1024 slots.
+constexpr int kFinalThreads = 64 * kDiagSlots;
+constexpr int kFinalUnroll = 8;
+
+__global__ void __launch_bounds__(kFinalThreads)
     k_diag_final(const double *__restrict__ part, int nb, double lx, double ly,
                  double *__restrict__ out) {
-  const int q = threadIdx.x;
-  if (q >= kDiagSlots) return;
-  double v = part[q];
-  for (int b = 1; b < nb; b++) v = q == 0 ? fmax(v, part[(size_t)b * kDiagSlots + q]) : v + part[(size_t)b * kDiagSlots + q];
+  const int t = threadIdx.x, q = t % kDiagSlots;
+  const int n = nb * kDiagSlots;
+  auto join = [&](double x, double y) { return q == 0 ? fmax(x, y) : x + y; };
+  double acc = 0.;  // the maximum is one of absolute values
+  int k = t;
+  for (; k + (kFinalUnroll - 1) * kFinalThreads < n; k += kFinalUnroll * kFinalThreads) {
+    double v[kFinalUnroll];
+#pragma unroll
+    for (int u = 0; u < kFinalUnroll; u++) v[u] = part[k + u * kFinalThreads];
+#pragma unroll
+    for (int u = 0; u < kFinalUnroll; u++) acc = join(acc, v[u]);
+  }
+  for (; k < n; k += kFinalThreads) acc = join(acc, part[k]);
+  __shared__ double sums[kFinalThreads];
+  sums[t] = acc;
+  // halve the 64 sums of each slot kind (t / kDiagSlots counts them)
+  for (int half = 32; half > 0; half >>= 1) {
+    __syncthreads();
+    if (t / kDiagSlots < half) sums[t] = join(sums[t], sums[t + half * kDiagSlots]);
+  }
+  if (t >= kDiagSlots) return;
+  double v = sums[t];
   if (q == 7) v /= ly;
   if (q == 8 || q == 9) {
     v /= lx * ly;
@@ -177,7 +204,7 @@ void launch_diag(hipStream_t s, const Geo &g, const DiagArgs &a, double *part, d
                  double ly, double *out) {
   const int nb = diag_partials(g);
   hipLaunchKernelGGL(k_diag, dim3(nb), dim3(kDiagThreads), 0, s, g, a, part);
-  hipLaunchKernelGGL(k_diag_final, dim3(1), dim3(64), 0, s, part, nb, lx, ly, out);
+  hipLaunchKernelGGL(k_diag_final, dim3(1), dim3(kFinalThreads), 0, s, part, nb, lx, ly, out);
 }
 
 }  // namespace sns
