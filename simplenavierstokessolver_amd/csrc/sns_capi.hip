@@ -408,7 +408,11 @@ LaunchKey launch_key(int itot, int jtot, const snsg_launch &req) {
   const bool part = k.chunk > 1;
   // the width applies to interface systems of up to 256 rows
   const int SR = part ? jtot / k.chunk - 1 : 0;
-  k.cols = part && SR <= 256 ? (req.ysolve_cols ? req.ysolve_cols : ysolve_cols_rule(SR)) : 0;
+  const bool onepass =
+      part && ysolve_one_pass(itot, jtot, k.chunk, req.ysolve_cols, req.ysolve_recompute);
+  k.cols = part && !onepass && SR <= 256
+               ? (req.ysolve_cols ? req.ysolve_cols : ysolve_cols_rule(SR))
+               : 0;
   k.recompute = part ? req.ysolve_recompute : 0;
   k.split = req.split_corr;
   return k;
@@ -1110,6 +1114,9 @@ static YFactorArgs yfactor_args(const snsg_ctx *c, const Geo &g) {
   yf.L = yL;
   yf.S = yL ? g.jtot / yL : 0;
   yf.stride = yL ? (long)ysolve_table_doubles(yL) : 0;
+  yf.onepass =
+      yL && ysolve_one_pass(g.itot, g.jtot, yL, c->launch.ysolve_cols,
+                            c->launch.ysolve_recompute);
   return yf;
 }
 
@@ -1134,6 +1141,7 @@ static YArgs y_args(const snsg_ctx *c, const Geo &g, int rk, int f, const double
   y.qz = yL ? c->d_qz + (size_t)f * 3 * (g.jtot / yL) * g.itot : nullptr;
   y.cols = c->launch.ysolve_cols;
   y.recompute = c->launch.ysolve_recompute;
+  y.onepass = yL && ysolve_one_pass(g.itot, g.jtot, yL, y.cols, y.recompute);
   return y;
 }
 

@@ -94,11 +94,15 @@ struct YFactorArgs {
   double *out;
   int L, S;
   long stride;
+  int onepass;  // no factors of the reduced block (ysolve_one_pass)
 };
 // chunk length of the partitioned y solve for jtot rows (0: not applicable)
 int ysolve_chunk(int jtot);
 bool ysolve_chunk_ok(int jtot, int L);
 int ysolve_cols_rule(int SR);
+// whether the solve of jtot rows in chunks of L runs as one kernel, given the
+// launch shapes ysolve_cols and ysolve_recompute (0: the rule)
+bool ysolve_one_pass(int itot, int jtot, int L, int cols, int recompute);
 size_t ysolve_table_doubles(int L);
 void launch_yfactor(hipStream_t s, const YFactorArgs &a);
 void launch_yfactor_batch(hipStream_t s, const YFactorArgs *dev, int nz);

@@ -94,6 +94,7 @@ struct YArgs {
   // launch shapes of the partitioned solve (host side; 0: the rule):
   // columns per workgroup of the interface solve, 1 recompute / 2 store
   int cols, recompute;
+  int onepass;  // whole columns in one kernel (ysolve_one_pass)
 };
 
 // ---- boundary values (src/fluid/boundary_conditions.c, src/temperature/boundary_conditions.c)

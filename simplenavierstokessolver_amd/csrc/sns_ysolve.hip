@@ -18,7 +18,9 @@
 //     solved per column as the reference solves periodic systems
 //     (src/linalg.c:52-108): the (S-1)-row block with the right-hand side
 //     and with [-O, 0, .., 0, -O], then the last unknown, then the rest.
-// Three kernels: k_ylocal (the interior solves; the first and last interior
+// k_ycol does all of it in one kernel, a workgroup holding whole columns (the
+// rule's choice up to 256 chunks).  Otherwise, three kernels: k_ylocal
+// (the interior solves; the first and last interior
 // values of each chunk go to qz rows S..3S-1), k_yreduced (the interface
 // system, one wave per column, into qz rows 0..S-1), k_yapply (the
 // corrections and out = in + x with boundary values).  When there are
@@ -26,9 +28,9 @@
 // bit for bit the same, instead of reading them back: a few flops per cell
 // for 32 instead of 40 bytes per cell.  Otherwise k_ylocal also stores the
 // interior solution and k_yapply_rows applies it row by row (one thread per
-// cell, which keeps small instances busy).  The factors of T and of the reduced system depend on
-// dt; k_yfactor computes them once per step for the three substages and
-// fields.  Rounding differs from the reference's sequential sweep at the
+// cell, which keeps small instances busy).  The factors of T and of the
+// reduced system depend on dt; k_yfactor computes them once per step for the
+// three substages and fields.  Rounding differs from the reference's sequential sweep at the
 // ulp level.
 #include "sns_launch.h"
 #include "sns_fast.h"
@@ -61,11 +63,14 @@ bool ysolve_chunk_ok(int jtot, int L) {
 }
 
 size_t ysolve_table_doubles(int L) {
-  return kYHead + 3 * (size_t)(L - 1) + 4 * (size_t)(kYRedNT * kYRedM);
+  (void)L;
+  return kYHead + 4 * (size_t)kYMaxL + 4 * (size_t)(kYRedNT * kYRedM);
 }
 
-// Table of one (substage, field): header [lambda, c, D, O, den, 0, 0, 0],
-// the interior factors r, beta and the spike v (L-1 entries each), then the
+// Table of one (substage, field): header [lambda, c, D, O, den, a, g, K] (a, g,
+// K: the interface kernel of k_ycol),
+// the interior factors r, beta, the spike v and its reverse (L-1 entries each,
+// zeros up to kYMaxL), then the
 // reduced (S-1)-row block's interleaved LU tables r, al, be (sns_lu.h) and
 // its matrix-only solution q1 in the same layout.
 struct YTab {
@@ -74,11 +79,14 @@ struct YTab {
   __device__ __forceinline__ double lambda() const { return p[0]; }
   __device__ __forceinline__ double O() const { return p[3]; }
   __device__ __forceinline__ double den() const { return p[4]; }
+  __device__ __forceinline__ double decay() const { return p[5]; }
+  __device__ __forceinline__ double green() const { return p[6]; }
+  __device__ __forceinline__ int doublings() const { return (int)p[7]; }
   __device__ __forceinline__ const double *r() const { return p + kYHead; }
-  __device__ __forceinline__ const double *beta() const { return p + kYHead + L1; }
-  __device__ __forceinline__ const double *v() const { return p + kYHead + 2 * L1; }
+  __device__ __forceinline__ const double *beta() const { return p + kYHead + kYMaxL; }
+  __device__ __forceinline__ const double *v() const { return p + kYHead + 2 * kYMaxL; }
   __device__ __forceinline__ const double *red(int k) const {
-    return p + kYHead + 3 * L1 + (size_t)k * kYRedNT * kYRedM;
+    return p + kYHead + 4 * kYMaxL + (size_t)k * kYRedNT * kYRedM;
   }
 };
 
@@ -106,7 +114,8 @@ __global__ void __launch_bounds__(64) k_yfactor(S src) {
   const int s = blockIdx.x, f = blockIdx.y;
   const int L1 = a.L - 1, SR = a.S - 1;  // interior rows; rows of the reduced block
   double *t = a.out + (size_t)(s * 3 + f) * a.stride;
-  for (int k = threadIdx.x; k < NR; k += 64) srr[k] = sal[k] = sbe[k] = sq1[k] = 0.;
+  if (!a.onepass)
+    for (int k = threadIdx.x; k < NR; k += 64) srr[k] = sal[k] = sbe[k] = sq1[k] = 0.;
   __syncthreads();
   if (threadIdx.x == 0) {
     const double gam = s == 0 ? a.gamma[0] : s == 1 ? a.gamma[1] : a.gamma[2];
@@ -135,44 +144,58 @@ __global__ void __launch_bounds__(64) k_yfactor(S src) {
     const double lam2 = lam * lam;
     const double D = c - lam2 * sv[0] - lam2 * sv[0];
     const double O = -(lam2 * sv[L1 - 1]);
-    // reduced (S-1)-row block: interleaved factors (row k at lu_slot), and
-    // q1, the block's solution for the right-hand side [-O, 0, .., 0, -O]:
-    // its forward sweep in the same loop, both carried in registers
-    auto slot = [](int k) { return (k % kYRedM) * kYRedNT + k / kYRedM; };
-    double rp = 0., bp = 0., yq = 0.;
-    for (int k = 0; k < SR; k++) {
-      const double piv = k == 0 ? D : D - O * bp;
-      rp = 1. / piv;
-      bp = O * rp;
-      const double alk = k == 0 ? 0. : -(rp * O);
-      srr[slot(k)] = rp;
-      sal[slot(k)] = alk;
-      sbe[slot(k)] = k == SR - 1 ? 0. : -bp;
-      const double rhs = (k == 0 ? -O : 0.) + (k == SR - 1 ? -O : 0.);
-      yq = rp * rhs + alk * yq;
-      sq1[slot(k)] = yq;
-    }
-    double xq = sq1[slot(SR - 1)];
-    for (int k = SR - 2; k >= 0; k--) {
-      xq = sq1[slot(k)] + sbe[slot(k)] * xq;
-      sq1[slot(k)] = xq;
-    }
     shead[0] = lam;
     shead[1] = c;
     shead[2] = D;
     shead[3] = O;
-    shead[4] = D + O * sq1[slot(0)] + O * sq1[slot(SR - 1)];
-    shead[5] = shead[6] = shead[7] = 0.;
+    // the inverse of the cyclic system (see k_ycol): entries g a^|k| summed
+    // over the periods, D > 2|O|; K doublings leave a tail below 2^-60
+    const double Om = fabs(O), disc = sqrt((D - 2. * Om) * (D + 2. * Om));
+    const double dec = 2. * Om / (D + disc);
+    int K = 0;
+    for (double pk = dec; pk > 0x1p-60 * (1. - dec) && K < 40; K++) pk *= pk;
+    shead[5] = dec;
+    shead[6] = 1. / disc;
+    shead[7] = (double)K;
+    if (a.onepass) {
+      shead[4] = 0.;
+    } else {
+      // reduced (S-1)-row block: interleaved factors (row k at lu_slot), and
+      // q1, the block's solution for the right-hand side [-O, 0, .., 0, -O]:
+      // its forward sweep in the same loop, both carried in registers
+      auto slot = [](int k) { return (k % kYRedM) * kYRedNT + k / kYRedM; };
+      double rp = 0., bp = 0., yq = 0.;
+      for (int k = 0; k < SR; k++) {
+        const double piv = k == 0 ? D : D - O * bp;
+        rp = 1. / piv;
+        bp = O * rp;
+        const double alk = k == 0 ? 0. : -(rp * O);
+        srr[slot(k)] = rp;
+        sal[slot(k)] = alk;
+        sbe[slot(k)] = k == SR - 1 ? 0. : -bp;
+        const double rhs = (k == 0 ? -O : 0.) + (k == SR - 1 ? -O : 0.);
+        yq = rp * rhs + alk * yq;
+        sq1[slot(k)] = yq;
+      }
+      double xq = sq1[slot(SR - 1)];
+      for (int k = SR - 2; k >= 0; k--) {
+        xq = sq1[slot(k)] + sbe[slot(k)] * xq;
+        sq1[slot(k)] = xq;
+      }
+      shead[4] = D + O * sq1[slot(0)] + O * sq1[slot(SR - 1)];
+    }
   }
   __syncthreads();
-  double *r = t + kYHead, *beta = r + L1, *v = beta + L1;
-  double *rr = t + kYHead + 3 * L1, *al = rr + NR, *be = al + NR, *q1 = be + NR;
+  double *r = t + kYHead, *beta = r + kYMaxL, *v = beta + kYMaxL, *w = v + kYMaxL;
+  double *rr = w + kYMaxL, *al = rr + NR, *be = al + NR, *q1 = be + NR;
   if (threadIdx.x < kYHead) t[threadIdx.x] = shead[threadIdx.x];
-  for (int m = threadIdx.x; m < L1; m += 64) {
-    r[m] = sr[m];
-    beta[m] = sbeta[m];
-    v[m] = sv[m];
+  for (int m = threadIdx.x; m < kYMaxL; m += 64) {
+    r[m] = m < L1 ? sr[m] : 0.;
+    beta[m] = m < L1 ? sbeta[m] : 0.;
+    v[m] = m < L1 ? sv[m] : 0.;
+    w[m] = m < L1 ? sv[L1 - 1 - m] : 0.;
   }
+  if (a.onepass) return;
   for (int k = threadIdx.x; k < NR; k += 64) {
     rr[k] = srr[k];
     al[k] = sal[k];
@@ -492,7 +515,169 @@ __global__ void __launch_bounds__(256) k_yapply(S src) {
   }
 }
 
+// ------------------------------------------- whole columns in one kernel
+
+// The solve of CW = 1 << lg adjacent columns by one workgroup, thread (s, c)
+// holding chunk s of column c in registers (LM >= L rows; the factors of the
+// rows past L-1 are 0).  The interior solves are those of k_ylocal.  The
+// cyclic interface system D p_s + O (p_{s-1} + p_{s+1}) = rhs_s has constant
+// coefficients, D > 2|O| and O < 0, so its inverse is known: with
+// a = 2|O| / (D + sqrt(D^2 - 4 O^2)) and g = 1/sqrt(D^2 - 4 O^2),
+//   p_s = g sum_k a^|k| rhs_{s+k}   (k over all integers, rhs periodic),
+// the product of the two one-sided sums' recurrences (D + O(E + 1/E) =
+// |O|/a (1 - aE)(1 - a/E), E the shift).  The sums double their length every
+// step, F_s += a^d F_{s-d} with d = 1, 2, 4, .., across the chunks in LDS,
+// both sides in the same steps; a falls geometrically with the chunk length,
+// so a handful of steps (k_yfactor's K) reach the tail below 2^-60.  Then
+// the corrections and out = in + x with boundary values as in k_yapply.
+//
+// Memory bounds it on large grids: increments and substage-start values are
+// read once and the result written once, 24 B per cell and field against 32
+// of the three kernels, with 16 to 32 loads in flight per thread; on small
+// ones it saves two launches and round trips through memory.  The fields
+// of a substage, three kernels before and this one now: 256x512 15.2 and 5.5
+// us (one field), 512x1024 26.2 and 12.5, 1024x2048 56 and 31, 2048x4096
+// 208 and 154 us (3.9 TB/s; its 1024 threads fill a CU, so loading,
+// solving and storing overlap only across CUs).
+template <int LM, class S>
+__global__ void __launch_bounds__(1024) k_ycol(S src, int lg) {
+  const YArgs a = src.get();
+  extern __shared__ double ylds[];
+  const int NT = blockDim.x, t = threadIdx.x;
+  double2 *fb = reinterpret_cast<double2 *>(ylds);  // [2][NT]
+  double *slast = ylds + 4 * NT, *sz = ylds + 5 * NT;
+  const int CW = 1 << lg, L = a.L, L1 = a.L - 1, nS = a.S, n = a.n;
+  const int c = t & (CW - 1), s = t >> lg;
+  const int col = xcd_remap(blockIdx.x, gridDim.x) * CW + c;
+  const int r0 = min(s, nS - 1) * L;  // first row (0-based) of the chunk
+  const int cc = min(col, n - 1);
+  // the factor table is read through the constant address space: scalar loads
+  const YTab tb{a.yfac, L1};
+  const __attribute__((address_space(4))) double *tr =
+      (const __attribute__((address_space(4))) double *)(uintptr_t)tb.r();
+  const auto *tbeta = tr + kYMaxL, *tv = tbeta + kYMaxL, *tw = tv + kYMaxL;
+  // row m of the chunk, rows past the last one repeating it
+  double x[LM];
+#pragma unroll
+  for (int m = 0; m < LM; m++)
+    x[m] = ldr(a.qf, (int)((unsigned)r0 * (unsigned)n + (unsigned)cc +
+                           (unsigned)min(m, L1) * (unsigned)n));
+  const double lam = tb.lambda();
+  // interior rows 1..L-1 with zero interface values
+  double y = 0.;
+#pragma unroll
+  for (int k = 0; k < LM - 1; k++) {
+    y = __builtin_fma(-tbeta[k], y, x[k + 1] * tr[k]);
+    x[k + 1] = y;
+  }
+#pragma unroll
+  for (int k = LM - 3; k >= 0; k--) x[k + 1] = __builtin_fma(-tbeta[k], x[k + 2], x[k + 1]);
+  double last = x[1];
+#pragma unroll
+  for (int k = 1; k < LM - 1; k++)
+    if (k == L1 - 1) last = x[k + 1];
+  // substage-start values of the first rows, in flight over the interface
+  // solve (out may be in: a thread loads its rows before it stores them, and
+  // no other thread reads them)
+  constexpr int G = LM < 16 ? LM : 16;
+  const bool ux = a.kind == KIND_UX;
+  const unsigned pitch = ux ? a.g.pu : a.g.pc;
+  const unsigned off = (unsigned)(r0 + 1) * pitch + (unsigned)cc + 1u;
+  double v[G];
+#pragma unroll
+  for (int k = 0; k < G; k++) v[k] = ldr(a.in, (int)(off + (unsigned)min(k, L1) * pitch));
+  slast[t] = last;
+  __syncthreads();
+  const int prev = s == 0 ? nS - 1 : s - 1, next = s + 1 >= nS ? 0 : s + 1;
+  const double rhs = x[0] - lam * (slast[(prev << lg) + c] + x[1]);
+  double F = rhs, B = rhs, p = tb.decay();
+  const int K = tb.doublings();
+  int d = 1;
+  for (int k = 0; k < K; k++) {
+    double2 *b = fb + (k & 1) * NT;
+    b[t] = make_double2(F, B);
+    __syncthreads();
+    const int sm = s - d < 0 ? s - d + nS : s - d, sp = s + d >= nS ? s + d - nS : s + d;
+    F = __builtin_fma(p, b[(sm << lg) + c].x, F);
+    B = __builtin_fma(p, b[(sp << lg) + c].y, B);
+    p *= p;
+    d = 2 * d >= nS ? 2 * d - nS : 2 * d;
+  }
+  const double zs = tb.green() * (F + (B - rhs));
+  sz[t] = zs;
+  __syncthreads();
+  const double zn = sz[(next << lg) + c];
+  if (s >= nS || col >= n) return;
+  const double ls = lam * zs, ln = lam * zn;
+  x[0] = zs;
+#pragma unroll
+  for (int k = 0; k < LM - 1; k++)
+    x[k + 1] = __builtin_fma(-ls, tv[k], __builtin_fma(-ln, tw[k], x[k + 1]));
+  double *o = a.out;
+#pragma unroll
+  for (int m0 = 0; m0 < LM; m0 += G) {
+    if (m0) {
+#pragma unroll
+      for (int k = 0; k < G; k++)
+        if (m0 + k < LM) v[k] = ldr(a.in, (int)(off + (unsigned)min(m0 + k, L1) * pitch));
+    }
+#pragma unroll
+    for (int k = 0; k < G; k++) {
+      const int m = m0 + k;
+      if (m >= LM || m > L1) continue;
+      const double val = v[k] + x[m];
+      str(o, (int)(off + (unsigned)m * pitch), val);
+      // periodic copies of rows 1 and jtot
+      if (m == 0 && s == 0) str(o, (int)((unsigned)(a.g.jtot + 1) * pitch + cc + 1u), val);
+      if (m == L1 && s == nS - 1) str(o, cc + 1, val);
+    }
+  }
+  // wall values of the chunk's rows (and, but for T, of the halo rows)
+#pragma unroll
+  for (int side = 0; side < 2; side++) {
+    if (col != (side ? n - 1 : 0)) continue;
+    const unsigned iw = side ? n + 1 : 0;
+    const bool temp = a.kind == KIND_TEMP;
+    const double wv = temp ? (side ? -0.5 : +0.5) : 0.;
+    for (int m = 0; m < L; m++) str(o, (int)((unsigned)(r0 + 1 + m) * pitch + iw), wv);
+    if (!temp && s == 0) str(o, (int)((unsigned)(a.g.jtot + 1) * pitch + iw), wv);
+    if (!temp && s == nS - 1) str(o, (int)iw, wv);
+  }
+}
+
 // ------------------------------------------------------------- launch
+
+// The one-kernel solve is the rule's choice where a workgroup of 1024
+// threads holds 8 columns (up to 128 chunks; 64-byte row segments), or 4 on
+// narrow grids, whose fields the caches hold: 4096x8192 IMP-IMP takes 8.49
+// ms/step with 4 columns against 8.20 in three kernels, 2048x8192 4.27 and
+// 4.26, 256x8192 0.651 and 0.730, 1024x4096 (8 columns) 1.09 and 1.22.
+// Explicit launch shapes of the interface solve or of the recompute choice,
+// and the environment variables that force them, keep the three kernels.
+// The rule depends on the grid and the shapes alone, so instances agree bit
+// for bit alone and in a batch.
+constexpr int kYColNarrow = 1024;  // widest grid that takes 4 columns
+
+bool ysolve_one_pass(int itot, int jtot, int L, int cols, int recompute) {
+  if (L < 4 || cols || recompute) return false;
+  if (jtot / L > (itot <= kYColNarrow ? 256 : 128)) return false;
+  for (const char *e : {"SNSG_YSOLVE_RECOMPUTE", "SNSG_YSOLVE_COLS", "SNSG_YSOLVE_CW"})
+    if (getenv(e)) return false;
+  return true;
+}
+
+// Columns per workgroup: 16 (rows of 128 bytes) where 1024 threads hold
+// them, fewer while that leaves CUs without a workgroup (no bit depends on
+// it).
+template <int LM, class S>
+static void ycol_launch(hipStream_t s, int n, int nS, S src, int nz) {
+  int lg = 4;
+  while ((nS << lg) > 1024) lg--;
+  while (lg > 2 && (size_t)((n + (1 << lg) - 1) >> lg) * nz < 256) lg--;
+  const int NT = ((nS << lg) + 63) / 64 * 64;
+  const dim3 g((n + (1 << lg) - 1) >> lg, 1, nz);
+  hipLaunchKernelGGL((k_ycol<LM, S>), g, dim3(NT), 6 * sizeof(double) * NT, s, src, lg);
+}
 
 // Chunk columns (threads of the per-chunk kernels) from which the interiors
 // are solved twice rather than stored: 4096 waves, unless the instance's
@@ -556,6 +741,13 @@ static int y_col_waves(int n) {
 
 template <class S>
 static void ypart(hipStream_t s, const YArgs &shape, int n, S src, int nz, int nrule) {
+  if (shape.onepass) {
+    if (shape.L <= 8) ycol_launch<8>(s, n, shape.S, src, nz);
+    else if (shape.L <= 16) ycol_launch<16>(s, n, shape.S, src, nz);
+    else if (shape.L <= 24) ycol_launch<24>(s, n, shape.S, src, nz);
+    else ycol_launch<32>(s, n, shape.S, src, nz);
+    return;
+  }
   const bool recompute = y_recompute((size_t)n * shape.S * nrule, shape.recompute);
   const int cw = y_col_waves(n);
   if (cw == 4) ylocal_launch<4>(s, n, shape.S, recompute, src, nz);

@@ -22,3 +22,33 @@ def test_diagnostics_partial_counts(sns, jtot):
                    ("nu_eps_k", nu[2]), ("nu_eps_h", nu[3])):
         assert abs(d[k] - ref) <= 1e-12 * abs(ref), (k, d[k], ref)
     inst.close()
+
+
+# (itot, jtot, dt, Ra): chunk lengths 4 to 32 (every register tile of the
+# kernel and its remainders), 4 to 256 chunks, 4 to 16 columns per workgroup
+# with ragged last tiles; lambda = pf/dy^2 from 1e-4 (no doubling step) to
+# 1e3 (the sums wrap around the period many times)
+YCOL_CASES = [
+    (8, 16, 1e-3, 1e8), (5, 16, 1.0, 1e2), (33, 45, 1e-2, 1e6), (19, 96, 1.0, 1e2),
+    (37, 200, 0.1, 1e4), (17, 324, 1e-2, 1e8), (12, 1000, 0.1, 1e4), (40, 960, 1e-3, 1e8),
+    (70, 2048, 1e-2, 1e6), (21, 4096, 1e-3, 1e6), (13, 8192, 1e-3, 1e4),
+]
+
+
+@pytest.mark.parametrize("case", YCOL_CASES)
+def test_ycol_against_oracle(sns, case):
+    """Crank-Nicolson in y by whole columns, T and both velocities, against
+    the oracle's sequential periodic sweeps.  The diagonal 1 + 2 lambda is
+    rounded to eps (1 + 2 lambda) while the smallest eigenvalue is 1, so two
+    correct solvers differ by a few eps (1 + 2 lambda)."""
+    itot, jtot, dt, Ra = case
+    o, inst = make_pair(sns, itot, jtot, 3.0, 0, 1, seed=31, dt=dt, Ra=Ra)
+    lam = 0.5 * dt * max(2.0 ** -0.5, 2.0 ** 0.5) / Ra ** 0.5 * (jtot / 2.0) ** 2
+    tol = 1e-13 + 32 * np.finfo(float).eps * (1 + 2 * lam)
+    o.update_temp(1)
+    inst.update_temp(1)
+    o.update_velocity(1)
+    inst.update_velocity(1)
+    for n in ("temp", "ux", "uy"):
+        assert_close(inst.download(n)[1:-1], o.f[n][1:-1], tol, n)
+    inst.close()
