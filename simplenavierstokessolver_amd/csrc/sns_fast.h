@@ -45,20 +45,30 @@ __device__ __forceinline__ double dv(double a, double b, double r) {
 
 // ---------------------------------------------------------- lane shifts
 
+// v moved between lanes by the DPP control CTRL; lanes without a source get
+// the bits of `none` (with none = 0 the hardware fills them: one instruction
+// per half).
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b & 0xffffffffll), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+template <int CTRL, int ROW_MASK = 0xf>
+__device__ __forceinline__ double dpp_f64(double v, double none) {
+  const long long b = __double_as_longlong(v), o = __double_as_longlong(none);
+  const int lo = __builtin_amdgcn_update_dpp((int)(unsigned)(o & 0xffffffffll),
+                                             (int)(unsigned)(b & 0xffffffffll), CTRL, ROW_MASK,
+                                             0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp((int)(o >> 32), (int)(b >> 32), CTRL, ROW_MASK, 0xf,
+                                             false);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
 // Value of v in lane l-1 (lane 0: 0).
-__device__ __forceinline__ double from_left(double v) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b & 0xffffffffll), 0x138, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x138, 0xf, 0xf, false);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
+__device__ __forceinline__ double from_left(double v) { return dpp_f64<0x138>(v); }
 // Value of v in lane l+1 (lane 63: 0).
-__device__ __forceinline__ double from_right(double v) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b & 0xffffffffll), 0x130, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x130, 0xf, 0xf, false);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
+__device__ __forceinline__ double from_right(double v) { return dpp_f64<0x130>(v); }
 // Per-column tables, all indexed like the reference arrays they derive from
 // (entry I-1 holds the value for column I unless noted).  They live in one
 // allocation of 14 double tables and one of 4 double2 tables, each table

@@ -19,6 +19,7 @@
 // [k*NT + t], so that the loads of a wave are contiguous.
 #pragma once
 #include <hip/hip_runtime.h>
+#include "sns_fast.h"
 
 namespace sns {
 
@@ -117,56 +118,88 @@ struct LuTabLUr {
   }
 };
 
-// composition of affine maps x -> A x + B: (A2,B2) after (A1,B1)
-__device__ __forceinline__ void aff_after(double &A, double &B, double A1, double B1) {
-  B = A * B1 + B;
-  A = A * A1;
+// Exclusive scan over the threads of a workgroup of the affine maps
+// x -> A x + B[f], NF of them with one common A (forward: thread t receives
+// the composition of maps 0..t-1 applied to 0; reverse: of maps NT-1..t+1).
+// Within a wave the maps are composed across 1, 2, 4 and 8 lanes of each row
+// of 16 by DPP, then across the rows; then one map per wave through LDS.  The
+// scan is a chain of latencies (a DPP step is a few cycles, a bpermute an LDS
+// round trip): with all six steps by bpermute, and A scanned once per f, the
+// x solves of the Poisson equation took 5.7 us at 128x192, 9.0 at 512x1024 and
+// 131 at 4096x8192, now 4.4, 7.0 and 112.
+// scr holds (1 + NF)*(NT/64) doubles; the caller orders any later write of
+// scr after the reads here (another scan uses other scratch, and the callers'
+// next LDS phase starts behind a barrier of their own).
+template <int CTRL, int NF>
+__device__ __forceinline__ void affine_step(double &A, double (&B)[NF]) {
+  const double Ao = dpp_f64<CTRL>(A, 1.);
+#pragma unroll
+  for (int f = 0; f < NF; f++) B[f] = __builtin_fma(A, dpp_f64<CTRL>(B[f]), B[f]);
+  A *= Ao;
+}
+template <int CTRL, int ROW_MASK, int NF>
+__device__ __forceinline__ void affine_bcast(double &A, double (&B)[NF]) {
+  const double Ao = dpp_f64<CTRL, ROW_MASK>(A, 1.);
+#pragma unroll
+  for (int f = 0; f < NF; f++)
+    B[f] = __builtin_fma(A, dpp_f64<CTRL, ROW_MASK>(B[f], 0.), B[f]);
+  A *= Ao;
 }
 
-// Exclusive affine scan over the threads of a workgroup (forward: thread t
-// receives the composition of maps 0..t-1 applied to 0; reverse: of maps
-// NT-1..t+1).  NF independent scans share the barriers.  scr holds
-// 2*NF*(NT/64) doubles; the caller orders any later write of scr after the
-// reads here (another scan uses other scratch, and the callers' next LDS
-// phase starts behind a barrier of their own).
 template <int NT, int NF, bool REVERSE>
-__device__ __forceinline__ void affine_scan_excl(double (&A)[NF], double (&B)[NF], double (&C)[NF],
+__device__ __forceinline__ void affine_scan_excl(double A, double (&B)[NF], double (&C)[NF],
                                                  double *scr) {
   constexpr int NW = NT / 64;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  // inclusive scan inside the wave
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if constexpr (!REVERSE) {
+    affine_step<0x111>(A, B);  // row_shr 1, 2, 4, 8
+    affine_step<0x112>(A, B);
+    affine_step<0x114>(A, B);
+    affine_step<0x118>(A, B);
+    affine_bcast<0x142, 0xa>(A, B);  // lane 15 of rows 0, 2 to rows 1, 3
+    affine_bcast<0x143, 0xc>(A, B);  // lane 31 to rows 2, 3
+  } else {
+    affine_step<0x101>(A, B);  // row_shl 1, 2, 4, 8
+    affine_step<0x102>(A, B);
+    affine_step<0x104>(A, B);
+    affine_step<0x108>(A, B);
+    // first lane of rows 1, 3 to rows 0, 2, then lane 32 to rows 0, 1
 #pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
+    for (int half = 16; half <= 32; half *= 2) {
+      const int src = (lane & ~(2 * half - 1)) | half;
+      const bool ok = !(lane & half);
+      const double Ao = __shfl(A, src);
 #pragma unroll
-    for (int f = 0; f < NF; f++) {
-      const double Ao = REVERSE ? __shfl_down(A[f], off) : __shfl_up(A[f], off);
-      const double Bo = REVERSE ? __shfl_down(B[f], off) : __shfl_up(B[f], off);
-      const bool ok = REVERSE ? (lane + off < 64) : (lane >= off);
-      if (ok) aff_after(A[f], B[f], Ao, Bo);
+      for (int f = 0; f < NF; f++) {
+        const double Bo = __shfl(B[f], src);
+        B[f] = ok ? __builtin_fma(A, Bo, B[f]) : B[f];
+      }
+      A = ok ? A * Ao : A;
     }
   }
-  // wave totals
-  const int last = REVERSE ? 0 : 63;
-  if (lane == last) {
+  double cin[NF];
 #pragma unroll
-    for (int f = 0; f < NF; f++) {
-      scr[(f * NW + wave) * 2 + 0] = A[f];
-      scr[(f * NW + wave) * 2 + 1] = B[f];
+  for (int f = 0; f < NF; f++) cin[f] = 0.;
+  if constexpr (NW > 1) {
+    // wave totals
+    double *w0 = scr + wave * (1 + NF);
+    if (lane == (REVERSE ? 0 : 63)) {
+      w0[0] = A;
+#pragma unroll
+      for (int f = 0; f < NF; f++) w0[1 + f] = B[f];
+    }
+    __syncthreads();
+    for (int k = 0; k < (REVERSE ? NW - 1 - wave : wave); k++) {
+      const double *w = scr + (REVERSE ? NW - 1 - k : k) * (1 + NF);
+#pragma unroll
+      for (int f = 0; f < NF; f++) cin[f] = __builtin_fma(w[0], cin[f], w[1 + f]);
     }
   }
-  __syncthreads();
 #pragma unroll
   for (int f = 0; f < NF; f++) {
-    double cin = 0.;
-    if (!REVERSE) {
-      for (int w = 0; w < wave; w++) cin = scr[(f * NW + w) * 2] * cin + scr[(f * NW + w) * 2 + 1];
-    } else {
-      for (int w = NW - 1; w > wave; w--) cin = scr[(f * NW + w) * 2] * cin + scr[(f * NW + w) * 2 + 1];
-    }
-    const double incl = A[f] * cin + B[f];  // value after this thread's map
-    const double prev = REVERSE ? __shfl_down(incl, 1) : __shfl_up(incl, 1);
-    const bool edge = REVERSE ? (lane == 63) : (lane == 0);
-    C[f] = edge ? cin : prev;
+    const double incl = __builtin_fma(A, cin[f], B[f]);  // value after this thread's map
+    const double prev = REVERSE ? from_right(incl) : from_left(incl);
+    C[f] = lane == (REVERSE ? 63 : 0) ? cin[f] : prev;
   }
 }
 
@@ -177,7 +210,7 @@ __device__ __forceinline__ void affine_scan_excl(double (&A)[NF], double (&B)[NF
 template <int NT, int M, int NS, class TAB = LuTab>
 __device__ __forceinline__ void lu_solve_shared(double (&d)[NS][M], const TAB &tab,
                                                 double *scr) {
-  double A[NS], B[NS], C[NS];
+  double B[NS], C[NS];
   double P[M];
   {
     double y[NS];
@@ -191,17 +224,14 @@ __device__ __forceinline__ void lu_solve_shared(double (&d)[NS][M], const TAB &t
       P[k] = pr;
 #pragma unroll
       for (int s = 0; s < NS; s++) {
-        y[s] = r * d[s][k] + al * y[s];
+        y[s] = __builtin_fma(al, y[s], r * d[s][k]);
         d[s][k] = y[s];
       }
     }
 #pragma unroll
-    for (int s = 0; s < NS; s++) {
-      A[s] = P[M - 1];
-      B[s] = y[s];
-    }
+    for (int s = 0; s < NS; s++) B[s] = y[s];
   }
-  affine_scan_excl<NT, NS, false>(A, B, C, scr);
+  affine_scan_excl<NT, NS, false>(P[M - 1], B, C, scr);
   double Q[M];
   {
     double x[NS];
@@ -215,22 +245,18 @@ __device__ __forceinline__ void lu_solve_shared(double (&d)[NS][M], const TAB &t
       Q[k] = pr;
 #pragma unroll
       for (int s = 0; s < NS; s++) {
-        d[s][k] += P[k] * C[s];
-        x[s] = d[s][k] + be * x[s];
+        x[s] = __builtin_fma(be, x[s], __builtin_fma(P[k], C[s], d[s][k]));
         d[s][k] = x[s];
       }
     }
 #pragma unroll
-    for (int s = 0; s < NS; s++) {
-      A[s] = Q[0];
-      B[s] = x[s];
-    }
+    for (int s = 0; s < NS; s++) B[s] = x[s];
   }
-  affine_scan_excl<NT, NS, true>(A, B, C, scr + 2 * NS * (NT / 64));
+  affine_scan_excl<NT, NS, true>(Q[0], B, C, scr + (1 + NS) * (NT / 64));
 #pragma unroll
   for (int s = 0; s < NS; s++)
 #pragma unroll
-    for (int k = 0; k < M; k++) d[s][k] += Q[k] * C[s];
+    for (int k = 0; k < M; k++) d[s][k] = __builtin_fma(Q[k], C[s], d[s][k]);
 }
 
 }  // namespace sns

@@ -3,7 +3,7 @@ smallest and largest of a range), each against the CPU oracle."""
 import numpy as np
 import pytest
 
-from test_gpu_parity import assert_close, make_pair
+from test_gpu_parity import assert_close, interior, make_pair, pinned_gauge  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
@@ -51,4 +51,20 @@ def test_ycol_against_oracle(sns, case):
     inst.update_velocity(1)
     for n in ("temp", "ux", "uy"):
         assert_close(inst.download(n)[1:-1], o.f[n][1:-1], tol, n)
+    inst.close()
+
+
+@pytest.mark.parametrize("itot", [4, 63, 64, 65, 256, 257, 512, 513, 1024, 1025, 2049, 4097])
+def test_x_solves_at_row_widths(sns, pinned_gauge, itot):  # noqa: F811
+    """The affine scans of the x solves at one lane, one wave and the edges of
+    every row width (threads x unknowns per thread): the implicit-x update of
+    T to the bar of the sequential sweep (1e-13) and the potential to 1e-11
+    after removing its mean, as the other sizes are held to."""
+    o, inst = make_pair(sns, itot, 8, float(itot), 1, 0, seed=itot)
+    o.update_temp(1)
+    inst.update_temp(1)
+    assert_close(inst.download("temp"), o.f["temp"], 1e-13, "temp")
+    o.compute_potential(1)
+    inst.compute_potential(1)
+    assert_close(interior(inst.download("psi")), interior(o.f["psi"]), 1e-11, "psi", demean=True)
     inst.close()
