@@ -621,10 +621,10 @@ static int cnx_solve(snsg_ctx *c, int kind, int rkstep, const double *srca, cons
                      const double *srcg, double *field, double *qout) {
   const Geo &g = c->geo;
   int rc;
-  if (!lu_row_threads(g.itot))
+  if (!pred_impx_supported(g.itot))
     return set_err(SNSG_E_SIZE, "implicit x needs itot <= 8192");
   if (!c->d_lu) {
-    c->lu_ntm = lu_table_entries(g.itot);
+    c->lu_ntm = lu_table_entries(g.itot, g.jtot);
     if ((rc = ctx_alloc((void **)&c->d_lu, sizeof(double) * lu_table_doubles(c->lu_ntm),
                         &c->mem)))
       return rc;
@@ -911,7 +911,7 @@ extern "C" int snsg_instance_bytes(const snsg_config *cfg, size_t *bytes) {
     const int L = launch_key((int)itot, (int)jtot, tuned_launch((int)itot, (int)jtot)).chunk;
     if (L > 1) n += d * 9 * ysolve_table_doubles(L) + 9 * d * (jtot / L) * itot;
   }
-  if (cfg->implicitx) n += d * lu_table_doubles(lu_table_entries((int)itot));
+  if (cfg->implicitx) n += d * lu_table_doubles(lu_table_entries((int)itot, (int)jtot));
   Geo g{};
   g.itot = (int)itot;
   g.jtot = (int)jtot;
@@ -1158,7 +1158,7 @@ int step_prepare(snsg_ctx *c) {
   }
   if ((rc = ysolve_prepare(c))) return rc;
   if (c->treat.implicitx && !c->d_lu) {
-    c->lu_ntm = lu_table_entries(itot);
+    c->lu_ntm = lu_table_entries(itot, jtot);
     if ((rc = ctx_alloc((void **)&c->d_lu, sizeof(double) * lu_table_doubles(c->lu_ntm), &c->mem))) return rc;
   }
   if (!c->d_part) {

@@ -168,6 +168,30 @@ __device__ __forceinline__ Rows3 c_rows(const Geo &g, const double *f, int j) {
 // lanes and rows) feed it.  Operation order follows the reference
 // expression by expression.
 
+// Split of the diffusive terms dif1 (x), dif2 (y) between the explicit part
+// A and the implicit part G.  IX, IY: the treatment of x and y where the
+// kernel knows it (1 implicit, 0 explicit), so the terms with weight 0 are
+// left out (they would add a zero) and weight 1 costs nothing; -1: the
+// weights are read.
+template <int IX = -1, int IY = -1>
+struct Weights {
+  double ex, ey, ix, iy;
+  __device__ __forceinline__ double a(double adv, double dif1, double dif2) const {
+    if constexpr (IX < 0) return adv + ex * dif1 + ey * dif2;
+    double v = adv;
+    if constexpr (IX == 0) v += dif1;
+    if constexpr (IY == 0) v += dif2;
+    return v;
+  }
+  __device__ __forceinline__ double g(double dif1, double dif2) const {
+    if constexpr (IX < 0) return +ix * dif1 + iy * dif2;
+    if constexpr (IX == 1 && IY == 1) return dif1 + dif2;
+    else if constexpr (IX == 1) return dif1;
+    else if constexpr (IY == 1) return dif2;
+    else return 0.;
+  }
+};
+
 // Temperature at (i, j) and its neighbours, with the velocities it is
 // advected by: src/temperature/update.c:33-84
 struct TempPt {
@@ -187,11 +211,10 @@ struct CellX {
 // dtdx_xp = (T(i+1)-T(i))/DXC(i+1), are given (the t_xm, t_xp entries of v
 // are not read): a kernel holding consecutive columns forms each face
 // gradient once and hands it to both cells.
-template <bool P2 = false>
+template <bool P2 = false, class W>
 __device__ __forceinline__ void temp_src_g(const Geo &g, const Tables &tb, const CellX &x,
                                            const TempPt &v, double dtdx_xm, double dtdx_xp,
-                                           double wex, double wey, double wix, double wiy,
-                                           double &srca, double &srcg) {
+                                           const W &w, double &srca, double &srcg) {
   const double dy = tb.dy, rdy = tb.rdy;
   const double dtdy_ym = dv<P2>(-v.t_ym + v.t_c, dy, rdy);
   const double dtdy_yp = dv<P2>(-v.t_c + v.t_yp, dy, rdy);
@@ -199,17 +222,17 @@ __device__ __forceinline__ void temp_src_g(const Geo &g, const Tables &tb, const
   const double adv2 = -0.5 * v.uy_c * dtdy_ym - 0.5 * v.uy_p * dtdy_yp;
   const double dif1 = dv<P2>(g.kappa_T * (dtdx_xp - dtdx_xm), x.dxf, x.rdxf);
   const double dif2 = dv<P2>(g.kappa_T * (dtdy_yp - dtdy_ym), dy, rdy);
-  srca = +(adv1 + adv2) + wex * dif1 + wey * dif2;
-  srcg = +wix * dif1 + wiy * dif2;
+  srca = w.a(+(adv1 + adv2), dif1, dif2);
+  srcg = w.g(dif1, dif2);
 }
 
-template <bool LANE = false, bool P2 = false>
+template <bool LANE = false, bool P2 = false, class W>
 __device__ __forceinline__ void temp_src_v(const Geo &g, const Tables &tb, const CellX &x,
-                                           const TempPt &v, double wex, double wey, double wix,
-                                           double wiy, double &srca, double &srcg) {
+                                           const TempPt &v, const W &w, double &srca,
+                                           double &srcg) {
   const double dtdx_xp = dv<P2>(-v.t_c + v.t_xp, x.dxc_p, x.rdxc_p);
   const double dtdx_xm = LANE ? from_left(dtdx_xp) : dv<P2>(-v.t_xm + v.t_c, x.dxc, x.rdxc);
-  temp_src_g<P2>(g, tb, x, v, dtdx_xm, dtdx_xp, wex, wey, wix, wiy, srca, srcg);
+  temp_src_g<P2>(g, tb, x, v, dtdx_xm, dtdx_xp, w, srca, srcg);
 }
 
 // x-momentum at face (i, j), i = 2..itot: src/fluid/update_velocity.c:34-101
@@ -226,11 +249,10 @@ struct FaceX {
 };
 // The x-gradients (UX(i)-UX(i-1))/DXF(i-1) and (UX(i+1)-UX(i))/DXF(i) are
 // given, as for temp_src_g (u_xm and u_xp still enter the interpolations).
-template <bool P2 = false>
+template <bool P2 = false, class W>
 __device__ __forceinline__ void ux_src_g(const Geo &g, const Tables &tb, const FaceX &x,
                                          const UxPt &v, double duxdx_xm, double duxdx_xp,
-                                         double wex, double wey, double wix, double wiy,
-                                         double &srca, double &srcg) {
+                                         const W &w, double &srca, double &srcg) {
   const double dy = tb.dy, rdy = tb.rdy;
   const double duxdy_ym = dv<P2>(-v.u_ym + v.u_c, dy, rdy);
   const double duxdy_yp = dv<P2>(-v.u_c + v.u_yp, dy, rdy);
@@ -243,18 +265,18 @@ __device__ __forceinline__ void ux_src_g(const Geo &g, const Tables &tb, const F
   const double dif1 = dv<P2>(g.kappa_u * (duxdx_xp - duxdx_xm), x.dxc, x.rdxc);
   const double dif2 = dv<P2>(g.kappa_u * (duxdy_yp - duxdy_ym), dy, rdy);
   const double pre = dv<P2>(-(v.p_c - v.p_m), x.dxc, x.rdxc);
-  srca = +(adv1 + adv2) + wex * dif1 + wey * dif2 + v.tf;
-  srcg = +wix * dif1 + wiy * dif2 + pre;
+  srca = w.a(+(adv1 + adv2), dif1, dif2) + v.tf;
+  srcg = w.g(dif1, dif2) + pre;
 }
 
-template <bool LANE = false, bool P2 = false>
+template <bool LANE = false, bool P2 = false, class W>
 __device__ __forceinline__ void ux_src_v(const Geo &g, const Tables &tb, const FaceX &x,
-                                         const UxPt &v, double wex, double wey, double wix,
-                                         double wiy, double &srca, double &srcg) {
+                                         const UxPt &v, const W &w, double &srca,
+                                         double &srcg) {
   const double duxdx_xp = dv<P2>(-v.u_c + v.u_xp, x.dxf, x.rdxf);
   const double duxdx_xm =
       LANE ? from_left(duxdx_xp) : dv<P2>(-v.u_xm + v.u_c, x.dxf_m, x.rdxf_m);
-  ux_src_g<P2>(g, tb, x, v, duxdx_xm, duxdx_xp, wex, wey, wix, wiy, srca, srcg);
+  ux_src_g<P2>(g, tb, x, v, duxdx_xm, duxdx_xp, w, srca, srcg);
 }
 
 // y-momentum at (i, j), i = 1..itot: src/fluid/update_velocity.c:128-189
@@ -265,11 +287,10 @@ struct UyPt {
 };
 // The x-gradients (UY(i)-UY(i-1))/DXC(i) and (UY(i+1)-UY(i))/DXC(i+1) are
 // given, as for temp_src_g.
-template <bool P2 = false>
+template <bool P2 = false, class W>
 __device__ __forceinline__ void uy_src_g(const Geo &g, const Tables &tb, const CellX &x,
                                          const UyPt &v, double duydx_xm, double duydx_xp,
-                                         double wex, double wey, double wix, double wiy,
-                                         double &srca, double &srcg) {
+                                         const W &w, double &srca, double &srcg) {
   const double dy = tb.dy, rdy = tb.rdy;
   const double duydy_ym = dv<P2>(-v.v_ym + v.v_c, dy, rdy);
   const double duydy_yp = dv<P2>(-v.v_c + v.v_yp, dy, rdy);
@@ -282,17 +303,17 @@ __device__ __forceinline__ void uy_src_g(const Geo &g, const Tables &tb, const C
   const double dif1 = dv<P2>(g.kappa_u * (duydx_xp - duydx_xm), x.dxf, x.rdxf);
   const double dif2 = dv<P2>(g.kappa_u * (duydy_yp - duydy_ym), dy, rdy);
   const double pre = dv<P2>(-(v.p_c - v.p_ym), dy, rdy);
-  srca = +(adv1 + adv2) + wex * dif1 + wey * dif2;
-  srcg = +wix * dif1 + wiy * dif2 + pre;
+  srca = w.a(+(adv1 + adv2), dif1, dif2);
+  srcg = w.g(dif1, dif2) + pre;
 }
 
-template <bool LANE = false, bool P2 = false>
+template <bool LANE = false, bool P2 = false, class W>
 __device__ __forceinline__ void uy_src_v(const Geo &g, const Tables &tb, const CellX &x,
-                                         const UyPt &v, double wex, double wey, double wix,
-                                         double wiy, double &srca, double &srcg) {
+                                         const UyPt &v, const W &w, double &srca,
+                                         double &srcg) {
   const double duydx_xp = dv<P2>(-v.v_c + v.v_xp, x.dxc_p, x.rdxc_p);
   const double duydx_xm = LANE ? from_left(duydx_xp) : dv<P2>(-v.v_xm + v.v_c, x.dxc, x.rdxc);
-  uy_src_g<P2>(g, tb, x, v, duydx_xm, duydx_xp, wex, wey, wix, wiy, srca, srcg);
+  uy_src_g<P2>(g, tb, x, v, duydx_xm, duydx_xp, w, srca, srcg);
 }
 
 // ------------------------------------------------ loaders (pointer form)
@@ -314,7 +335,7 @@ __device__ __forceinline__ void temp_src_t(const Geo &g, const Tables &tb, const
   const TempPt v = {ldr(temp.c, i), ldr(temp.c, i - 1), ldr(temp.c, i + 1), ldr(temp.m, i),
                     ldr(temp.p, i), ldr(ux.c, i - 1),   ldr(ux.c, i),       ldr(uy.c, i),
                     ldr(uy.p, i)};
-  temp_src_v<false, P2>(g, tb, cell_x(tb, i), v, wex, wey, wix, wiy, srca, srcg);
+  temp_src_v<false, P2>(g, tb, cell_x(tb, i), v, Weights<>{wex, wey, wix, wiy}, srca, srcg);
 }
 
 template <bool P2 = false>
@@ -325,7 +346,7 @@ __device__ __forceinline__ void ux_src_t(const Geo &g, const Tables &tb, const R
   const UxPt v = {ldr(ux.c, i - 1), ldr(ux.c, i - 2), ldr(ux.c, i), ldr(ux.m, i - 1),
                   ldr(ux.p, i - 1), ldr(uy.c, i - 1), ldr(uy.c, i), ldr(uy.p, i - 1),
                   ldr(uy.p, i),     ldr(p.c, i),      ldr(p.c, i - 1), tf};
-  ux_src_v<false, P2>(g, tb, face_x(tb, i), v, wex, wey, wix, wiy, srca, srcg);
+  ux_src_v<false, P2>(g, tb, face_x(tb, i), v, Weights<>{wex, wey, wix, wiy}, srca, srcg);
 }
 
 template <bool P2 = false>
@@ -336,7 +357,7 @@ __device__ __forceinline__ void uy_src_t(const Geo &g, const Tables &tb, const R
   const UyPt v = {ldr(uy.c, i),     ldr(uy.c, i - 1), ldr(uy.c, i + 1), ldr(uy.m, i),
                   ldr(uy.p, i),     ldr(ux.m, i - 1), ldr(ux.c, i - 1), ldr(ux.m, i),
                   ldr(ux.c, i),     ldr(p.c, i),      ldr(p.m, i)};
-  uy_src_v<false, P2>(g, tb, cell_x(tb, i), v, wex, wey, wix, wiy, srca, srcg);
+  uy_src_v<false, P2>(g, tb, cell_x(tb, i), v, Weights<>{wex, wey, wix, wiy}, srca, srcg);
 }
 
 // ---------------------------------------------------------------- stores
@@ -437,6 +458,16 @@ __device__ __forceinline__ int xcd_remap(int b, int nblocks) {
   const int per = nblocks / NX, rem = nblocks % NX;
   const int xcd = b % NX, slot = b / NX;
   return xcd * per + (xcd < rem ? xcd : rem) + slot;
+}
+
+// The same in runs: `per` consecutive work items on one XCD, the next `per`
+// on the next, so the XCDs work on neighbouring runs; the rest after the last
+// full round of the 8 XCDs in hardware order.
+__device__ __forceinline__ int xcd_groups(int b, int nblocks, int per) {
+  const int round = 8 * per;
+  if (b >= nblocks / round * round) return b;
+  const int r = b % round;
+  return b - r + (r % 8) * per + r / 8;
 }
 
 }  // namespace sns

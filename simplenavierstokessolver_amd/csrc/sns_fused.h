@@ -58,9 +58,36 @@ struct DtArgs {
 // bit for bit, and that triple (lu_table_doubles in all)
 constexpr int kLuHdr = 4;
 inline size_t lu_table_doubles(int ntm) { return 27 * (size_t)ntm + 9 * kLuHdr; }
-// threads of the row kernels for itot (the tables interleave lu_table_entries
-// = threads x 8 unknowns per thread); 0 where itot is not supported
-int lu_row_threads(int itot);
+// Threads NT and unknowns per thread M of the row kernels of an itot x jtot
+// grid (the tables interleave NT*M entries); NT = 0 where itot is not
+// supported
+struct RowShape {
+  int NT, M;
+};
+RowShape row_shape(int itot, int jtot);
+
+// Launch FN<NT, M>(args) of the row shapes in use: M = 8 up to 1024 threads, M
+// = 4 up to 256, M = 2 up to 256
+#define SNS_ROW_DISPATCH(SHAPE, CALL)                                                  \
+  do {                                                                                 \
+    const RowShape rs_ = (SHAPE);                                                      \
+    if (rs_.M == 2) {                                                                  \
+      if (rs_.NT == 64) { CALL(64, 2); }                                               \
+      else if (rs_.NT == 128) { CALL(128, 2); }                                        \
+      else { CALL(256, 2); }                                                           \
+    } else if (rs_.M == 4) {                                                           \
+      if (rs_.NT == 64) { CALL(64, 4); }                                               \
+      else if (rs_.NT == 128) { CALL(128, 4); }                                        \
+      else { CALL(256, 4); }                                                           \
+    } else {                                                                           \
+      if (rs_.NT == 64) { CALL(64, 8); }                                               \
+      else if (rs_.NT == 128) { CALL(128, 8); }                                        \
+      else if (rs_.NT == 256) { CALL(256, 8); }                                        \
+      else if (rs_.NT == 512) { CALL(512, 8); }                                        \
+      else { CALL(1024, 8); }                                                          \
+    }                                                                                  \
+  } while (0)
+
 
 // Crank-Nicolson in x on the reference layouts (the per-function entry
 // points): the increment of each row from the RK sources (or qin), solved
@@ -115,7 +142,7 @@ void launch_ypart_fields_batch(hipStream_t s, const YArgs &shape, const YArgs *d
                                int nf);
 
 bool pred_impx_supported(int itot);
-int lu_table_entries(int itot);
+int lu_table_entries(int itot, int jtot);
 void launch_lu_factor(hipStream_t s, const LuFactorArgs &a);
 // predictor of one substage; a.lu, a.ntm: the LU tables when implicitx
 void launch_pred(hipStream_t s, const PredArgs &a, int implicitx);

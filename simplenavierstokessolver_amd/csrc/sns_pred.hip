@@ -3,21 +3,26 @@
 //
 // k_pred_rows evaluates, for one field and two adjacent rows per workgroup,
 // the source terms and RK increments of src/temperature/update.c:11-122 and
-// src/fluid/update_velocity.c:11-229, then solves the Crank-Nicolson system
-// in x of both rows (src/temperature/update.c:124-156,
+// src/fluid/update_velocity.c:11-229 (sns_rows.h), then solves the
+// Crank-Nicolson system in x of both rows (src/temperature/update.c:124-156,
 // src/fluid/update_velocity.c:231-270, 381-414) with the shared LU tables.
 //
-// Memory traffic is set by the number of load instructions, so neighbours
-// are not loaded twice:
-//  * x neighbours come from the adjacent lane (DPP wave shifts); each wave
-//    covers 62 columns and its first and last lanes only hold the halo
-//    values of the columns on either side;
-//  * the y neighbours of one row are the centre values of the other, and the
-//    per-column metrics and the LU tables serve both rows.
+// What bounds it on large grids is neither the HBM bytes (88 B per cell; 4.0
+// TB/s at 4096x8192) nor the arithmetic, but the way from the L2: the three
+// fields' workgroups read 18 rows for each row, and a run of columns that
+// does not start on a cache line costs a line more.  Evaluating one block of
+// a wave's own contiguous columns after the other, so that the lines at the
+// block ends were fetched twice, took 0.96 ms where the waves of a workgroup
+// side by side take 0.80; loads issued a block ahead did not help.  With one
+// column per lane and unrolled blocks (15900 instructions, 1700 of them moving
+// spilled scalars) it took 0.93.  us per launch, before and now: 4096x8192
+// 925 and 800, folded 1285 and 1067; 2048x4096 244 and 189; 1537x3000 163 and
+// 143; 512x1024 24.4 and 18.1; 225x360 13.8 and 9.8, folded 16.9 and 11.4.
 #include "sns_launch.h"
 #include "sns_fast.h"
 #include "sns_fused.h"
 #include "sns_lu.h"
+#include "sns_rows.h"
 
 namespace sns {
 
@@ -202,380 +207,151 @@ struct PredRowsLds {
 
 template <int M>
 __device__ __forceinline__ int pad_idx(int r) {
-  return r + r / M;
+  return r + (int)((unsigned)r / M);
 }
 
-constexpr int kWaveCols = 62;  // output columns per wave (lanes 1..62)
+// Stencil blocks: kBlockCols adjacent columns, two per lane (sns_rows.h), lanes
+// 0 and 63 holding the neighbours.  Block k of wave w is number k*NW + w of the
+// row, so the waves of a workgroup work side by side and share the cache lines
+// at the block ends while those are in L1.
+constexpr int kBlockCols = 124;
 
-// Lane position of stencil block k: unknown index ii (lanes 1..62 of each
-// wave own a column, lanes 0 and 63 hold the neighbours), the column i and
-// the clamped element indices of the cell arrays (ci), ux (ui), the column
-// tables (ti) and the RK history (hi).
-struct LanePos {
-  int ii, i, ci, ui, ti, hi;
-  bool out;
-  bool interior;  // all 64 lanes of the wave on columns 2..itot-1 (wave-uniform)
-};
-
-__device__ __forceinline__ LanePos lane_pos(int k, int nw, int i0, int n, int itot) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  LanePos p;
-  p.ii = (k * nw + wave) * kWaveCols + lane - 1;
-  p.i = p.ii + i0;
-  p.out = lane >= 1 && lane <= kWaveCols && p.ii < n;
-  p.ci = clampi(p.i, 0, itot + 1);
-  p.ui = clampi(p.i - 1, 0, itot);
-  p.ti = clampi(p.i - 1, 0, itot + 1);
-  p.hi = clampi(p.ii, 0, n - 1);
-  const int c0 = (k * nw + wave) * kWaveCols - 1 + i0;  // column of lane 0
-  p.interior = c0 >= 2 && c0 + 63 <= itot - 1;
-  return p;
+template <int NW>
+__device__ __forceinline__ LanePos block_pos(int k, int i0, int n, int itot) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  return lane_pos(1 + (k * NW + wave) * kBlockCols - 2, i0, n, itot, 0, n, 1, 63);
 }
 
-// The values one lane loads for the two rows of field F (0: T, 1: ux,
-// 2: uy): the substage-start fields around rows ja, jb, the column tables
-// and the RK history.
-template <int F>
-struct Raw;
-template <>
-struct Raw<0> {
-  double t_am, t_a, t_b, t_bp, u_a, u_b, v_a, v_b, v_bp, ba, bb;
-  double2 c2, f2, w2;
-};
-template <>
-struct Raw<1> {
-  double u_am, u_a, u_b, u_bp, v_a, v_b, v_bp, p_a, p_b, t_a, t_b, ba, bb;
-  double2 c2, f2, w2;
-};
-template <>
-struct Raw<2> {
-  double v_am, v_a, v_b, v_bp, u_am, u_a, u_b, p_am, p_a, p_b, ba, bb;
-  double2 c2, f2, w2;
-};
+// LDS slots of a lane's two unknowns; unknowns that are not the block's own go
+// to the unused slot after the first chunk.
+template <int M>
+__device__ __forceinline__ void lds_slots(const LanePos &p, int &s0, int &s1) {
+  s0 = p.out0 ? pad_idx<M>(p.ii) : M;
+  s1 = p.out1 ? pad_idx<M>(p.ii + 1) : M;
+}
 
-template <int F>
-__device__ __forceinline__ Raw<F> raw_load(const PredArgs &a, const LanePos &p, int ja, int jb,
-                                           int n) {
-  const Geo &g = a.g;
-  const Tables &tb = a.tb;
-  const size_t wc = (size_t)g.pc, wu = (size_t)g.pu;
-  const double *T = a.temp, *U = a.ux, *V = a.uy, *P = a.p;
-  Raw<F> r;
-  const double *H = F == 0 ? a.hist_t : (F == 1 ? a.hist_ux : a.hist_uy);
-  r.ba = a.read_hist ? ldr(H + (size_t)(ja - 1) * n, p.hi) : 0.;
-  r.bb = a.read_hist ? ldr(H + (size_t)(jb - 1) * n, p.hi) : 0.;
-  if (p.interior && tb.uniform) {
-    r.c2 = make_double2(tb.u_dxc, tb.u_rdxc);
-    r.f2 = make_double2(tb.u_dxf, tb.u_rdxf);
-    const double w = F == 1 ? tb.u_cU : tb.u_cT;
-    r.w2 = make_double2(w, w);
-  } else {
-    r.c2 = ldr2(tb.dxc2(), p.ti);
-    r.f2 = ldr2(tb.dxf2(), p.ti);
-    r.w2 = ldr2(F == 1 ? tb.cU2() : tb.cT2(), p.ti);
+// Whether a block has lanes with one own column: the first ux block (its
+// pairs start at face 1, which is none) and the last block of an odd row end.
+template <int F, int NW>
+__device__ __forceinline__ bool block_edge(int k, int n) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int b = k * NW + wave;
+  return (F == 1 && b == 0) || (b + 1) * kBlockCols >= n;
+}
+
+// The nk stencil blocks of one wave.
+template <int F, int NT, int M, bool P2, bool FOLD, int IMY>
+__device__ __forceinline__ void pred_stencils(const PredArgs &a, const RowSrc<F, FOLD> &q,
+                                              PredRowsLds<NT, M> &L, int ja, int jb,
+                                              bool write_a, int n, int i0, double dt,
+                                              int nk) {
+  const int itot = a.g.itot;
+#pragma unroll 1
+  for (int k = 0; k < nk; k++) {
+    const LanePos p = block_pos<NT / 64>(k, i0, n, itot);
+    const bool edge = block_edge<F, NT / 64>(k, n);
+    Raw<F> r;
+    double2 da, db;
+    raw_load<F, P2, FOLD, 0>(a.tb, q, p, r);
+    if constexpr (FOLD) raw_fold<F, P2, 1, 0, 0>(a, q, p, ja, jb, write_a, edge, dt, r);
+    raw_eval<F, P2, 1, IMY, 0>(a, q, r, p, write_a, edge, dt, da);
+    __builtin_amdgcn_sched_barrier(0);
+    raw_load<F, P2, FOLD, 1>(a.tb, q, p, r);
+    if constexpr (FOLD) raw_fold<F, P2, 1, 0, 1>(a, q, p, ja, jb, write_a, edge, dt, r);
+    raw_eval<F, P2, 1, IMY, 1>(a, q, r, p, write_a, edge, dt, db);
+    int s0, s1;
+    lds_slots<M>(p, s0, s1);
+    L.d[0][s0] = da.x;
+    L.d[0][s1] = da.y;
+    L.d[1][s0] = db.x;
+    L.d[1][s1] = db.y;
   }
-  if constexpr (F == 0) {
-    r.t_am = ldr(T + (ja - 1) * wc, p.ci);
-    r.t_a = ldr(T + ja * wc, p.ci);
-    r.t_b = ldr(T + jb * wc, p.ci);
-    r.t_bp = ldr(T + (jb + 1) * wc, p.ci);
-    r.u_a = ldr(U + ja * wu, p.ui);
-    r.u_b = ldr(U + jb * wu, p.ui);
-    r.v_a = ldr(V + ja * wc, p.ci);
-    r.v_b = ldr(V + jb * wc, p.ci);
-    r.v_bp = ldr(V + (jb + 1) * wc, p.ci);
-  } else if constexpr (F == 1) {
-    r.u_am = ldr(U + (ja - 1) * wu, p.ui);
-    r.u_a = ldr(U + ja * wu, p.ui);
-    r.u_b = ldr(U + jb * wu, p.ui);
-    r.u_bp = ldr(U + (jb + 1) * wu, p.ui);
-    r.v_a = ldr(V + ja * wc, p.ci);
-    r.v_b = ldr(V + jb * wc, p.ci);
-    r.v_bp = ldr(V + (jb + 1) * wc, p.ci);
-    r.p_a = ldr(P + ja * wc, p.ci);
-    r.p_b = ldr(P + jb * wc, p.ci);
-    r.t_a = a.forcing ? ldr(T + ja * wc, p.ci) : 0.;
-    r.t_b = a.forcing ? ldr(T + jb * wc, p.ci) : 0.;
-  } else {
-    r.v_am = ldr(V + (ja - 1) * wc, p.ci);
-    r.v_a = ldr(V + ja * wc, p.ci);
-    r.v_b = ldr(V + jb * wc, p.ci);
-    r.v_bp = ldr(V + (jb + 1) * wc, p.ci);
-    r.u_am = ldr(U + (ja - 1) * wu, p.ui);
-    r.u_a = ldr(U + ja * wu, p.ui);
-    r.u_b = ldr(U + jb * wu, p.ui);
-    r.p_am = ldr(P + (ja - 1) * wc, p.ci);
-    r.p_a = ldr(P + ja * wc, p.ci);
-    r.p_b = ldr(P + jb * wc, p.ci);
-  }
-  return r;
 }
 
-// The previous substage's correction applied to the values raw_load took
-// from its ux*, uy* and pressure, with the operations of k_corr (proj_* of
-// sns_fast.h; P2 gives the same bits as its divisions): psi of the rows the
-// corrected values need is loaded here, its x neighbours come from the
-// adjacent lanes.  Lane 0 of a ux workgroup loads psi(i-1) itself, since
-// the face and the pressure it corrects feed lane 1; in the other
-// workgroups lane 0 only feeds uy and T, which need no x neighbour of psi.
-//
-// Faces 2..itot and cells 1..itot are corrected, the rest keep what the
-// predictor stored, which is what k_corr leaves there:
-//  * faces: psi's wall columns are exact copies of its columns 1 and itot,
-//    so psi(i) - psi(i-1) is +0 at the wall faces 1 and itot+1 (and at the
-//    clamped lanes past them) and the correction leaves those faces as they
-//    are, with no select;
-//  * uy: the wall columns 0 and itot+1 are kept by a select in the uy
-//    workgroup, the only one whose outputs read them;
-//  * p: values outside cells 1..itot feed no output.
-// Row ja-2 of a uy workgroup wraps to jtot-1 for ja = 1 (periodic in y), and
-// its pressure of row 0 is taken from row jtot: ux*, uy* and psi carry
-// periodic copies in their halo rows, the pressure only once k_corr has
-// written it.  The uy workgroup stores the corrected pressure of its rows in
-// p_out, the stores of k_corr for those cells.
-template <int F, bool P2>
-__device__ __forceinline__ void raw_fold(const PredArgs &a, const LanePos &p, int ja, int jb,
-                                         bool write_a, double dt, Raw<F> &r) {
-  const Geo &g = a.g;
-  const Tables &tb = a.tb;
-  const int itot = g.itot;
-  const size_t wc = (size_t)g.pc;
-  const double *S = a.psi;
-  const double gdt = a.corr_gamma * dt;
-  const double fac = -gdt / g.two_Re;
-  const double rdxc = r.c2.y;  // 1./DXC(i)
-  const double dy = tb.dy, rdy = tb.rdy;
-  const int imx = a.tr.implicitx, imy = a.tr.implicity;
-  const double s_am = ldr(S + (size_t)(ja - 1) * wc, p.ci);
-  const double s_a = ldr(S + (size_t)ja * wc, p.ci);
-  const double s_b = ldr(S + (size_t)jb * wc, p.ci);
-  const double s_bp = ldr(S + (size_t)(jb + 1) * wc, p.ci);
-  // Lane shifts run on every lane, never under a divergent condition (a
-  // shift there would read the inactive neighbour lanes as 0).
-  if constexpr (F == 0) {
-    r.u_a = proj_ux(r.u_a, s_a, from_left(s_a), gdt, rdxc);
-    r.u_b = proj_ux(r.u_b, s_b, from_left(s_b), gdt, rdxc);
-    r.v_a = proj_uy<P2>(r.v_a, s_a, s_am, gdt, dy, rdy);
-    r.v_b = proj_uy<P2>(r.v_b, s_b, s_a, gdt, dy, rdy);
-    r.v_bp = proj_uy<P2>(r.v_bp, s_bp, s_b, gdt, dy, rdy);
-  } else {
-    const ProjX x = {r.c2.x, r.c2.y, from_right(r.c2.x), from_right(r.c2.y), r.f2.x, r.f2.y};
+// The substage-start values of the own field in rows ja, jb (corrected as in
+// raw_fold when folded), read again: the rows are in the caches since the
+// stencil phase, and the registers that would hold them (40 a thread) are
+// worth more there.
+template <int F, bool P2, bool FOLD>
+__device__ __forceinline__ void own_load(const PredArgs &a, const RowSrc<F, FOLD> &q,
+                                         const LanePos &p, double dt, double2 &oa, double2 &ob) {
+  const Buf &f = F == 0 ? q.T : F == 1 ? q.U : q.V;
+  oa = F == 1 ? bld2(f, p.u, q.u_a) : bld2(f, p.c, q.c_a);
+  ob = F == 1 ? bld2(f, p.u, q.u_b) : bld2(f, p.c, q.c_b);
+  if constexpr (FOLD && F != 0) {
+    const double gdt = a.corr_gamma * dt;
+    const double2 s_a = bld2(q.S, p.c, q.c_a), s_b = bld2(q.S, p.c, q.c_b);
     if constexpr (F == 1) {
-      const int cw = clampi(p.i - 1, 0, itot + 1);
-      double w_am = from_left(s_am), w_a = from_left(s_a), w_b = from_left(s_b),
-             w_bp = from_left(s_bp);
-      if ((threadIdx.x & 63) == 0) {
-        w_am = ldr(S + (size_t)(ja - 1) * wc, cw);
-        w_a = ldr(S + (size_t)ja * wc, cw);
-        w_b = ldr(S + (size_t)jb * wc, cw);
-        w_bp = ldr(S + (size_t)(jb + 1) * wc, cw);
-      }
-      const double e_a = from_right(s_a), e_b = from_right(s_b);
-      r.u_am = proj_ux(r.u_am, s_am, w_am, gdt, rdxc);
-      r.u_a = proj_ux(r.u_a, s_a, w_a, gdt, rdxc);
-      r.u_b = proj_ux(r.u_b, s_b, w_b, gdt, rdxc);
-      r.u_bp = proj_ux(r.u_bp, s_bp, w_bp, gdt, rdxc);
-      r.v_a = proj_uy<P2>(r.v_a, s_a, s_am, gdt, dy, rdy);
-      r.v_b = proj_uy<P2>(r.v_b, s_b, s_a, gdt, dy, rdy);
-      r.v_bp = proj_uy<P2>(r.v_bp, s_bp, s_b, gdt, dy, rdy);
-      r.p_a = proj_p<P2>(r.p_a, s_a, w_a, e_a, s_am, s_b, x, dy, rdy, fac, imx, imy);
-      r.p_b = proj_p<P2>(r.p_b, s_b, w_b, e_b, s_a, s_bp, x, dy, rdy, fac, imx, imy);
+      const double2 r = p.interior && a.tb.uniform
+                            ? make_double2(a.tb.u_rdxc, a.tb.u_rdxc)
+                            : bld2(q.tab, p.t, 3u * q.ts);
+      const double wa = from_left(s_a.y), wb = from_left(s_b.y);
+      oa = make_double2(proj_ux(oa.x, s_a.x, wa, gdt, r.x), proj_ux(oa.y, s_a.y, s_a.x, gdt, r.y));
+      ob = make_double2(proj_ux(ob.x, s_b.x, wb, gdt, r.x), proj_ux(ob.y, s_b.y, s_b.x, gdt, r.y));
     } else {
-      const bool cc = p.i >= 1 && p.i <= itot;  // uy cells the correction moves
-      const int jmm = ja >= 2 ? ja - 2 : g.jtot - 1;
-      const double s_amm = ldr(S + (size_t)jmm * wc, p.ci);
-      if (ja == 1) r.p_am = ldr(a.p + (size_t)g.jtot * wc, p.ci);
-      const double w_am = from_left(s_am), w_a = from_left(s_a), w_b = from_left(s_b);
-      const double e_am = from_right(s_am), e_a = from_right(s_a), e_b = from_right(s_b);
-      const double v_am = proj_uy<P2>(r.v_am, s_am, s_amm, gdt, dy, rdy);
-      const double v_a = proj_uy<P2>(r.v_a, s_a, s_am, gdt, dy, rdy);
-      const double v_b = proj_uy<P2>(r.v_b, s_b, s_a, gdt, dy, rdy);
-      const double v_bp = proj_uy<P2>(r.v_bp, s_bp, s_b, gdt, dy, rdy);
-      r.v_am = cc ? v_am : r.v_am;
-      r.v_a = cc ? v_a : r.v_a;
-      r.v_b = cc ? v_b : r.v_b;
-      r.v_bp = cc ? v_bp : r.v_bp;
-      r.u_am = proj_ux(r.u_am, s_am, w_am, gdt, rdxc);
-      r.u_a = proj_ux(r.u_a, s_a, w_a, gdt, rdxc);
-      r.u_b = proj_ux(r.u_b, s_b, w_b, gdt, rdxc);
-      r.p_am = proj_p<P2>(r.p_am, s_am, w_am, e_am, s_amm, s_a, x, dy, rdy, fac, imx, imy);
-      r.p_a = proj_p<P2>(r.p_a, s_a, w_a, e_a, s_am, s_b, x, dy, rdy, fac, imx, imy);
-      r.p_b = proj_p<P2>(r.p_b, s_b, w_b, e_b, s_a, s_bp, x, dy, rdy, fac, imx, imy);
-      if (p.out) {
-        if (write_a) put_c<1>(g, a.p_out, p.i, ja, r.p_a);
-        put_c<1>(g, a.p_out, p.i, jb, r.p_b);
-      }
+      const double2 s_am = bld2(q.S, p.c, q.c_am);
+      const double dy = a.tb.dy, rdy = a.tb.rdy;
+      oa = make_double2(proj_uy<P2>(oa.x, s_a.x, s_am.x, gdt, dy, rdy),
+                        proj_uy<P2>(oa.y, s_a.y, s_am.y, gdt, dy, rdy));
+      ob = make_double2(proj_uy<P2>(ob.x, s_b.x, s_a.x, gdt, dy, rdy),
+                        proj_uy<P2>(ob.y, s_b.y, s_a.y, gdt, dy, rdy));
     }
   }
 }
 
-// Source terms and RK increments of both rows from the loaded values (x
-// neighbours from the adjacent lanes); the new RK history is stored.
-template <int F, bool P2>
-__device__ __forceinline__ void raw_eval(const PredArgs &a, const Raw<F> &r, const LanePos &p,
-                                         int ja, int jb, int n, bool write_a, double dt,
-                                         double &da, double &db) {
-  const Geo &g = a.g;
-  const Tables &tb = a.tb;
-  const double wex = a.tr.w_ex_x, wey = a.tr.w_ex_y, wix = a.tr.w_im_x, wiy = a.tr.w_im_y;
-  double *H = F == 0 ? a.hist_t : (F == 1 ? a.hist_ux : a.hist_uy);
-  double *HA = H + (size_t)(ja - 1) * n, *HB = H + (size_t)(jb - 1) * n;
-  double A, G;
-  if constexpr (F == 0) {
-    CellX x;
-    x.dxc = r.c2.x;
-    x.rdxc = r.c2.y;
-    x.dxf = r.f2.x;
-    x.rdxf = r.f2.y;
-    x.c_xm = r.w2.x;
-    x.c_xp = r.w2.y;
-    x.dxc_p = from_right(x.dxc);
-    x.rdxc_p = from_right(x.rdxc);
-    const TempPt pa = {r.t_a, from_left(r.t_a), from_right(r.t_a), r.t_am, r.t_b,
-                       r.u_a, from_right(r.u_a), r.v_a, r.v_b};
-    const TempPt pb = {r.t_b, from_left(r.t_b), from_right(r.t_b), r.t_a, r.t_bp,
-                       r.u_b, from_right(r.u_b), r.v_b, r.v_bp};
-    temp_src_v<true, P2>(g, tb, x, pa, wex, wey, wix, wiy, A, G);
-    if (a.write_hist && p.out && write_a) str(HA, p.ii, A);
-    da = rk_incr(a.alpha, a.beta, a.gamma, dt, A, r.ba, G);
-    temp_src_v<true, P2>(g, tb, x, pb, wex, wey, wix, wiy, A, G);
-    if (a.write_hist && p.out) str(HB, p.ii, A);
-    db = rk_incr(a.alpha, a.beta, a.gamma, dt, A, r.bb, G);
-  } else if constexpr (F == 1) {
-    FaceX x;
-    x.dxf = r.f2.x;
-    x.rdxf = r.f2.y;
-    x.c_xm = r.w2.x;
-    x.c_xp = r.w2.y;
-    x.dxc = r.c2.x;
-    x.rdxc = r.c2.y;
-    x.dxf_m = from_left(x.dxf);
-    x.rdxf_m = from_left(x.rdxf);
-    double tf_a = 0., tf_b = 0.;
-    if (a.forcing) {
-      tf_a = 0.5 * from_left(r.t_a) + 0.5 * r.t_a;
-      tf_b = 0.5 * from_left(r.t_b) + 0.5 * r.t_b;
+// Final values in the blocks of the stencil phase: own + increment, or the
+// increment itself when a y solve follows (IMY).  rowa, rowb: byte offsets of
+// the rows in out; halo rows get copies where copy_* is set.
+template <int F, int NT, int M, bool P2, bool FOLD, int IMY>
+__device__ __forceinline__ void pred_emit(const PredArgs &a, const RowSrc<F, FOLD> &q,
+                                          const Buf &out, const PredRowsLds<NT, M> &L,
+                                          unsigned rowa, unsigned rowb, bool write_a,
+                                          bool copy_a, bool copy_b, unsigned top, int n, int i0,
+                                          double dt, int nk) {
+#pragma unroll 1
+  for (int k = 0; k < nk; k++) {
+    const LanePos p = block_pos<NT / 64>(k, i0, n, a.g.itot);
+    const bool edge = block_edge<F, NT / 64>(k, n);
+    int s0, s1;
+    lds_slots<M>(p, s0, s1);
+    double2 va = make_double2(L.d[0][s0], L.d[0][s1]);
+    double2 vb = make_double2(L.d[1][s0], L.d[1][s1]);
+    if constexpr (IMY) {
+      if (write_a) store_hist(out, p, edge, rowa, va);
+      store_hist(out, p, edge, rowb, vb);
+    } else {
+      double2 oa, ob;
+      own_load<F, P2, FOLD>(a, q, p, dt, oa, ob);
+      va = make_double2(oa.x + va.x, oa.y + va.y);
+      vb = make_double2(ob.x + vb.x, ob.y + vb.y);
+      const unsigned o = F == 1 ? p.u : p.c;
+      if (write_a) store_pair(out, p, edge, o, rowa, va);
+      store_pair(out, p, edge, o, rowb, vb);
+      if (copy_a) store_pair(out, p, edge, o, top, va);
+      if (copy_b) store_pair(out, p, edge, o, 0u, vb);
     }
-    const double v_bm = from_left(r.v_b);
-    const UxPt pa = {r.u_a, from_left(r.u_a), from_right(r.u_a), r.u_am, r.u_b,
-                     from_left(r.v_a), r.v_a, v_bm, r.v_b, r.p_a, from_left(r.p_a), tf_a};
-    const UxPt pb = {r.u_b, from_left(r.u_b), from_right(r.u_b), r.u_a, r.u_bp,
-                     v_bm, r.v_b, from_left(r.v_bp), r.v_bp, r.p_b, from_left(r.p_b), tf_b};
-    ux_src_v<true, P2>(g, tb, x, pa, wex, wey, wix, wiy, A, G);
-    if (a.write_hist && p.out && write_a) str(HA, p.ii, A);
-    da = rk_incr(a.alpha, a.beta, a.gamma, dt, A, r.ba, G);
-    ux_src_v<true, P2>(g, tb, x, pb, wex, wey, wix, wiy, A, G);
-    if (a.write_hist && p.out) str(HB, p.ii, A);
-    db = rk_incr(a.alpha, a.beta, a.gamma, dt, A, r.bb, G);
-  } else {
-    CellX x;
-    x.dxc = r.c2.x;
-    x.rdxc = r.c2.y;
-    x.dxf = r.f2.x;
-    x.rdxf = r.f2.y;
-    x.c_xm = r.w2.x;
-    x.c_xp = r.w2.y;
-    x.dxc_p = from_right(x.dxc);
-    x.rdxc_p = from_right(x.rdxc);
-    const double u_ap = from_right(r.u_a);
-    const UyPt pa = {r.v_a, from_left(r.v_a), from_right(r.v_a), r.v_am, r.v_b,
-                     r.u_am, r.u_a, from_right(r.u_am), u_ap, r.p_a, r.p_am};
-    const UyPt pb = {r.v_b, from_left(r.v_b), from_right(r.v_b), r.v_a, r.v_bp,
-                     r.u_a, r.u_b, u_ap, from_right(r.u_b), r.p_b, r.p_a};
-    uy_src_v<true, P2>(g, tb, x, pa, wex, wey, wix, wiy, A, G);
-    if (a.write_hist && p.out && write_a) str(HA, p.ii, A);
-    da = rk_incr(a.alpha, a.beta, a.gamma, dt, A, r.ba, G);
-    uy_src_v<true, P2>(g, tb, x, pb, wex, wey, wix, wiy, A, G);
-    if (a.write_hist && p.out) str(HB, p.ii, A);
-    db = rk_incr(a.alpha, a.beta, a.gamma, dt, A, r.bb, G);
-  }
-}
-
-// Blocks of kWaveCols columns per wave of the stencil phase: at most
-// ceil(ceil(NT*M / kWaveCols) / (NT/64)), 9 for M = 8.
-template <int NT, int M>
-constexpr int stencil_blocks() {
-  return ((NT * M + kWaveCols - 1) / kWaveCols + NT / 64 - 1) / (NT / 64);
-}
-
-// The workgroup's own field at rows ja, jb in Raw (the values the increments
-// are added to).
-template <int F>
-__device__ __forceinline__ double2 raw_own(const Raw<F> &r) {
-  if constexpr (F == 0) return make_double2(r.t_a, r.t_b);
-  else if constexpr (F == 1) return make_double2(r.u_a, r.u_b);
-  else return make_double2(r.v_a, r.v_b);
-}
-
-// Stencil phase of one workgroup: blocks K.. of the nk blocks per wave
-// (compile-time block index).  The workgroup's own field at rows ja, jb is
-// kept per block in own[] for the final values, so those rows are not read
-// a second time after the line solve.
-template <int K, int F, int NT, int M, bool P2, bool FOLD>
-__device__ __forceinline__ void pred_stencils(const PredArgs &a, PredRowsLds<NT, M> &L, int ja,
-                                              int jb, bool write_a, int n, int i0, double dt,
-                                              int nk, double2 (&own)[stencil_blocks<NT, M>()]) {
-  if constexpr (K < stencil_blocks<NT, M>()) {
-    if (K >= nk) return;
-    const LanePos p = lane_pos(K, NT / 64, i0, n, a.g.itot);
-    Raw<F> r = raw_load<F>(a, p, ja, jb, n);
-    if constexpr (FOLD) raw_fold<F, P2>(a, p, ja, jb, write_a, dt, r);
-    double da, db;
-    raw_eval<F, P2>(a, r, p, ja, jb, n, write_a, dt, da, db);
-    own[K] = raw_own<F>(r);
-    if (p.out) {
-      L.d[0][pad_idx<M>(p.ii)] = da;
-      L.d[1][pad_idx<M>(p.ii)] = db;
-    }
-    pred_stencils<K + 1, F, NT, M, P2, FOLD>(a, L, ja, jb, write_a, n, i0, dt, nk, own);
-  }
-}
-
-// Final values of blocks K.. of the stencil phase (compile-time block
-// index, so own[] stays in registers): own + increment with boundary values,
-// or the increment itself when a y solve follows.
-template <int K, int F, int NT, int M>
-__device__ __forceinline__ void pred_emit(const PredArgs &a, const PredRowsLds<NT, M> &L,
-                                          const double2 (&own)[stencil_blocks<NT, M>()], int ja,
-                                          int jb, bool write_a, int n, int i0, int nk) {
-  if constexpr (K < stencil_blocks<NT, M>()) {
-    if (K >= nk) return;
-    const LanePos p = lane_pos(K, NT / 64, i0, n, a.g.itot);
-    double *q = F == 0 ? a.q_t : (F == 1 ? a.q_u : a.q_v);
-    if (p.out) {
-#pragma unroll
-      for (int s = 0; s < 2; s++) {
-        if (s == 0 && !write_a) continue;
-        const int j = s == 0 ? ja : jb;
-        const double d = L.d[s][pad_idx<M>(p.ii)];
-        const double o = s == 0 ? own[K].x : own[K].y;
-        if (q) str(q + (size_t)(j - 1) * n, p.ii, d);
-        else if (F == 0) put_c<2>(a.g, a.out_t, p.i, j, o + d);
-        else if (F == 1) put_ux(a.g, a.out_u, p.i, j, o + d);
-        else put_c<0>(a.g, a.out_v, p.i, j, o + d);
-      }
-    }
-    pred_emit<K + 1, F, NT, M>(a, L, own, ja, jb, write_a, n, i0, nk);
   }
 }
 
 // One workgroup's field F for rows ja and jb (write_a: row ja is written):
 // stencils into LDS, the CN-x solve of both rows, final values.
-template <int F, int NT, int M, bool P2, bool FOLD>
+template <int F, int NT, int M, bool P2, bool FOLD, int IMY>
 __device__ __forceinline__ void pred_rows_body(const PredArgs &a, PredRowsLds<NT, M> &L, int ja,
                                                int jb, bool write_a) {
-  constexpr int NW = NT / 64;
-  constexpr int KB = stencil_blocks<NT, M>();
   const Geo &g = a.g;
   const int itot = g.itot;
   const int n = F == 1 ? itot - 1 : itot;
   const int i0 = F == 1 ? 2 : 1;
   const double dt = *a.dtp;
-  const int nk = ((n + kWaveCols - 1) / kWaveCols + NW - 1) / NW;
+  // stencil blocks of this wave that hold unknowns
+  constexpr int NW = NT / 64;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nb = (n + i0 - 1 + kBlockCols - 1) / kBlockCols;
+  const int nk = wave < nb ? (nb - wave + NW - 1) / NW : 0;
 
   // ---- stencils and RK increments of both rows into LDS (lane order)
-  double2 own[KB];
-  pred_stencils<0, F, NT, M, P2, FOLD>(a, L, ja, jb, write_a, n, i0, dt, nk, own);
+  const RowSrc<F, FOLD> q = row_src<F, FOLD>(a, ja, jb, n);
+  pred_stencils<F, NT, M, P2, FOLD, IMY>(a, q, L, ja, jb, write_a, n, i0, dt, nk);
   __syncthreads();
 
   // ---- Crank-Nicolson in x of both rows (chunk order)
@@ -602,38 +378,75 @@ __device__ __forceinline__ void pred_rows_body(const PredArgs &a, PredRowsLds<NT
 
   // ---- final values with boundary values, or the increments for a y
   // solve, in the lane order of the stencil phase
-  pred_emit<0, F, NT, M>(a, L, own, ja, jb, write_a, n, i0, nk);
+  const unsigned pitch = (unsigned)(IMY ? n : F == 1 ? g.pu : g.pc) * 8u;
+  const unsigned rows = (unsigned)(IMY ? g.jtot : g.jtot + 2);
+  double *dst = IMY ? (F == 0 ? a.q_t : F == 1 ? a.q_u : a.q_v)
+                    : (F == 0 ? a.out_t : F == 1 ? a.out_u : a.out_v);
+  const Buf out = IMY || F == 1 ? buf_of(dst, pitch * rows) : cell_buf(dst, pitch * rows);
+  const unsigned rowa = (unsigned)(IMY ? ja - 1 : ja) * pitch, rowb = rowa + pitch;
+  const unsigned top = (unsigned)(g.jtot + 1) * pitch;
+  const bool copy_a = !IMY && write_a && ja == 1, copy_b = !IMY && jb == g.jtot;
+  pred_emit<F, NT, M, P2, FOLD, IMY>(a, q, out, L, rowa, rowb, write_a, copy_a, copy_b, top, n,
+                                     i0, dt, nk);
+  if constexpr (!IMY) {
+    // wall values: both ends of both rows, one thread each
+    if (threadIdx.x < 4) {
+      const bool right = threadIdx.x & 1, second = threadIdx.x & 2;
+      const double wv = F != 0 ? 0. : right ? -0.5 : +0.5;
+      const unsigned wo = F == 1 ? (right ? (unsigned)itot * 8u : 0u)
+                                 : (right ? (unsigned)(itot + 2) * 8u : 8u);
+      if (second || write_a) bst(out, wo, second ? rowb : rowa, wv);
+      // halo rows: ux and uy only (T's walls end at rows 1 and jtot)
+      if (F != 0 && (second ? copy_b : copy_a)) bst(out, wo, second ? 0u : top, wv);
+    }
+  }
+}
+
+// Row pairs of one XCD's run before the next XCD's (xcd_groups): rows that
+// share neighbours meet in an L2, and the eight runs stay close in memory.
+// 2048x4096 IMP-IMP, us per launch: 234 with an eighth of the grid per XCD,
+// 232, 227, 226 and 224 with 1, 4, 8 and 64 pairs, 256 without any order.
+constexpr int kPredGroup = 64;
+
+// Waves per SIMD: the two rows' LDS leaves 4 (two workgroups per CU) at the
+// widest rows; the folded kernel with the division sequence needs 156
+// registers, so on narrower rows it takes 3 (1537x3000: 206 us, 220 with 4 and
+// spilled registers).
+template <bool P2, bool FOLD, int NT>
+constexpr int pred_waves() {
+  return FOLD && !P2 && NT <= 256 ? 3 : 4;
 }
 
 // Workgroup w: field w % nfld (+1 without the temperature equation) of rows
 // a = 2q+1 and b = a+1, q = w / nfld.  For odd jtot the last pair is shifted
 // down to (jtot-1, jtot) and writes row b only.  Consecutive w share an XCD.
-// FOLD: the fields are corrected as they are loaded (raw_fold).
-template <int NT, int M, bool P2, bool FOLD, class S>
-__global__ void __launch_bounds__(NT) k_pred_rows(S src, int nfld) {
+// FOLD: the fields are corrected as they are loaded (raw_fold).  IMY: a y
+// solve follows, the increments are the output.
+template <int NT, int M, bool P2, bool FOLD, int IMY, class S>
+__global__ void __launch_bounds__(NT, (pred_waves<P2, FOLD, NT>())) k_pred_rows(S src, int nfld) {
   const PredArgs a = src.get();
   extern __shared__ double lds_raw[];
   PredRowsLds<NT, M> &L = *reinterpret_cast<PredRowsLds<NT, M> *>(lds_raw);
-  const int w = xcd_remap(blockIdx.x, gridDim.x);
+  const int w = xcd_groups(blockIdx.x, gridDim.x, kPredGroup * nfld);
   const int q = w / nfld;
   const int f = w % nfld + (nfld == 3 ? 0 : 1);
   const int ja = min(2 * q + 1, a.g.jtot - 1), jb = ja + 1;
   const bool write_a = ja == 2 * q + 1;
-  if (f == 0) pred_rows_body<0, NT, M, P2, FOLD>(a, L, ja, jb, write_a);
-  else if (f == 1) pred_rows_body<1, NT, M, P2, FOLD>(a, L, ja, jb, write_a);
-  else pred_rows_body<2, NT, M, P2, FOLD>(a, L, ja, jb, write_a);
+  if (f == 0) pred_rows_body<0, NT, M, P2, FOLD, IMY>(a, L, ja, jb, write_a);
+  else if (f == 1) pred_rows_body<1, NT, M, P2, FOLD, IMY>(a, L, ja, jb, write_a);
+  else pred_rows_body<2, NT, M, P2, FOLD, IMY>(a, L, ja, jb, write_a);
 }
 
 // ---------------------------------------------------------------- launch
 
-template <int NT, int M, bool P2, bool FOLD, class S>
+template <int NT, int M, bool P2, bool FOLD, int IMY, class S>
 static void pred_rows_launch(hipStream_t s, const PredArgs &shape, S src, int nz) {
   const size_t lds = sizeof(PredRowsLds<NT, M>);
   static std::atomic<unsigned> attr{0};
-  lds_limit_once((const void *)k_pred_rows<NT, M, P2, FOLD, S>, lds, attr);
+  lds_limit_once((const void *)k_pred_rows<NT, M, P2, FOLD, IMY, S>, lds, attr);
   const int nfld = shape.with_temp ? 3 : 2;
   const int npair = (shape.g.jtot + 1) / 2;
-  hipLaunchKernelGGL((k_pred_rows<NT, M, P2, FOLD, S>), dim3(npair * nfld, 1, nz), dim3(NT), lds,
+  hipLaunchKernelGGL((k_pred_rows<NT, M, P2, FOLD, IMY, S>), dim3(npair * nfld, 1, nz), dim3(NT), lds,
                      s, src, nfld);
 }
 
@@ -642,78 +455,67 @@ static void lu_factor_launch(hipStream_t s, S src, int nz) {
   hipLaunchKernelGGL((k_lu_factor<NT, M, S>), dim3(3, 3, nz), dim3(NT), 0, s, src);
 }
 
-// (NT, M) of the row kernels for a given itot; ntm = NT*M >= itot
-static constexpr int kRowM = 8;
-static int row_config(int itot, int &NT, int &M) {
-  M = kRowM;
-  if (itot <= 64 * kRowM) NT = 64;
-  else if (itot <= 128 * kRowM) NT = 128;
-  else if (itot <= 256 * kRowM) NT = 256;
-  else if (itot <= 512 * kRowM) NT = 512;
-  else if (itot <= 1024 * kRowM) NT = 1024;
-  else return 0;
-  return NT * M;
+// Unknowns per thread: few where the rows' waves would leave SIMDs (1024)
+// without one or with one only, so that a wave evaluates one or two stencil
+// blocks instead of five and the substitutions are short; 8 where there are
+// waves enough, since every thread pays the scans.  Measured (us, M = 8, 4, 2):
+// 225x360 folded 14.4, 13.8, 11.4; 512x1024 19.9, 18.1, 20.1; 1024x2048 55.8,
+// 56.0 (M = 4); batches of three 128x256 11.8, 10.5, 10.2, of four 512x1024
+// 56.3, 59.4, 71.4.  It depends on the grid alone, so instances agree bit for
+// bit alone and in a batch.
+RowShape row_shape(int itot, int jtot) {
+  RowShape r{0, 8};
+  if (itot > 8192) return r;
+  const long rows = 3l * ((jtot + 1) / 2);
+  if (itot <= 512 && rows * ((itot + 127) / 128) <= 2048) r.M = 2;
+  else if (itot <= 1024 && rows * ((itot + 255) / 256) <= 4096) r.M = 4;
+  r.NT = 64;
+  while (r.NT * r.M < itot) r.NT *= 2;
+  return r;
 }
 
-bool pred_impx_supported(int itot) {
-  int NT, M;
-  return row_config(itot, NT, M) > 0;
-}
+bool pred_impx_supported(int itot) { return row_shape(itot, 4).NT > 0; }
 
-int lu_table_entries(int itot) {
-  int NT, M;
-  return row_config(itot, NT, M);
-}
-
-int lu_row_threads(int itot) {
-  int NT, M;
-  return row_config(itot, NT, M) ? NT : 0;
+int lu_table_entries(int itot, int jtot) {
+  const RowShape r = row_shape(itot, jtot);
+  return r.NT * r.M;
 }
 
 template <class S>
-static void lu_factor_dispatch(hipStream_t s, int itot, S src, int nz) {
-  int NT, M;
-  row_config(itot, NT, M);
-  switch (NT) {
-    case 64: lu_factor_launch<64, kRowM>(s, src, nz); break;
-    case 128: lu_factor_launch<128, kRowM>(s, src, nz); break;
-    case 256: lu_factor_launch<256, kRowM>(s, src, nz); break;
-    case 512: lu_factor_launch<512, kRowM>(s, src, nz); break;
-    default: lu_factor_launch<1024, kRowM>(s, src, nz); break;
-  }
+static void lu_factor_dispatch(hipStream_t s, const Geo &g, S src, int nz) {
+#define SNS_CALL(NT_, M_) lu_factor_launch<NT_, M_>(s, src, nz)
+  SNS_ROW_DISPATCH(row_shape(g.itot, g.jtot), SNS_CALL);
+#undef SNS_CALL
 }
 
 void launch_lu_factor(hipStream_t s, const LuFactorArgs &a) {
-  lu_factor_dispatch(s, a.g.itot, ArgOne<LuFactorArgs>{a}, 1);
+  lu_factor_dispatch(s, a.g, ArgOne<LuFactorArgs>{a}, 1);
 }
 
 void launch_lu_factor_batch(hipStream_t s, const LuFactorArgs &shape, const LuFactorArgs *dev,
                             int nz) {
-  lu_factor_dispatch(s, shape.g.itot, arg_batch<LuFactorArgs>(dev), nz);
+  lu_factor_dispatch(s, shape.g, arg_batch<LuFactorArgs>(dev), nz);
 }
 
-template <bool P2, bool FOLD, class S>
-static void pred_rows_select(hipStream_t s, const PredArgs &shape, S src, int nz, int NT) {
-  switch (NT) {
-    case 64: pred_rows_launch<64, kRowM, P2, FOLD>(s, shape, src, nz); break;
-    case 128: pred_rows_launch<128, kRowM, P2, FOLD>(s, shape, src, nz); break;
-    case 256: pred_rows_launch<256, kRowM, P2, FOLD>(s, shape, src, nz); break;
-    case 512: pred_rows_launch<512, kRowM, P2, FOLD>(s, shape, src, nz); break;
-    default: pred_rows_launch<1024, kRowM, P2, FOLD>(s, shape, src, nz); break;
-  }
+template <bool P2, bool FOLD, int IMY, class S>
+static void pred_rows_select(hipStream_t s, const PredArgs &shape, S src, int nz) {
+#define SNS_CALL(NT_, M_) pred_rows_launch<NT_, M_, P2, FOLD, IMY>(s, shape, src, nz)
+  SNS_ROW_DISPATCH(row_shape(shape.g.itot, shape.g.jtot), SNS_CALL);
+#undef SNS_CALL
 }
 
 // Power-of-two divisors select the kernel that divides by multiplying; a
 // psi argument the one that applies the previous substage's correction.
 template <class S>
 static void pred_rows_dispatch(hipStream_t s, const PredArgs &shape, S src, int nz) {
-  int NT, M;
-  row_config(shape.g.itot, NT, M);
   const bool p2 = pow2_division(shape.tb), fold = shape.psi != nullptr;
-  if (p2 && fold) pred_rows_select<true, true>(s, shape, src, nz, NT);
-  else if (p2) pred_rows_select<true, false>(s, shape, src, nz, NT);
-  else if (fold) pred_rows_select<false, true>(s, shape, src, nz, NT);
-  else pred_rows_select<false, false>(s, shape, src, nz, NT);
+  const bool imy = shape.tr.implicity;  // excludes fold
+  if (p2 && fold) pred_rows_select<true, true, 0>(s, shape, src, nz);
+  else if (p2 && imy) pred_rows_select<true, false, 1>(s, shape, src, nz);
+  else if (p2) pred_rows_select<true, false, 0>(s, shape, src, nz);
+  else if (fold) pred_rows_select<false, true, 0>(s, shape, src, nz);
+  else if (imy) pred_rows_select<false, false, 1>(s, shape, src, nz);
+  else pred_rows_select<false, false, 0>(s, shape, src, nz);
 }
 
 void launch_pred_rows(hipStream_t s, const PredArgs &a) {

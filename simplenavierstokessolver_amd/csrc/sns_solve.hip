@@ -124,9 +124,8 @@ __global__ void __launch_bounds__(NT) k_cnx_lu(CnxLuArgs a) {
   }
 }
 
-template <int KIND, int NT>
+template <int KIND, int NT, int M>
 static void cnx_lu_launch(hipStream_t s, const CnxLuArgs &a) {
-  constexpr int M = 8;
   const size_t lds = sizeof(double) * (NT * (M + 1) + 4 * (NT / 64));
   static std::atomic<unsigned> attr{0};
   lds_limit_once((const void *)k_cnx_lu<KIND, NT, M>, lds, attr);
@@ -135,13 +134,9 @@ static void cnx_lu_launch(hipStream_t s, const CnxLuArgs &a) {
 
 template <int KIND>
 static void cnx_lu_dispatch(hipStream_t s, const CnxLuArgs &a) {
-  switch (lu_row_threads(a.g.itot)) {
-    case 64: cnx_lu_launch<KIND, 64>(s, a); break;
-    case 128: cnx_lu_launch<KIND, 128>(s, a); break;
-    case 256: cnx_lu_launch<KIND, 256>(s, a); break;
-    case 512: cnx_lu_launch<KIND, 512>(s, a); break;
-    default: cnx_lu_launch<KIND, 1024>(s, a); break;
-  }
+#define SNS_CALL(NT_, M_) cnx_lu_launch<KIND, NT_, M_>(s, a)
+  SNS_ROW_DISPATCH(row_shape(a.g.itot, a.g.jtot), SNS_CALL);
+#undef SNS_CALL
 }
 
 void launch_cnx_lu(hipStream_t s, int kind, const CnxLuArgs &a) {

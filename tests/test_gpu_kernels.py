@@ -68,3 +68,42 @@ def test_x_solves_at_row_widths(sns, pinned_gauge, itot):  # noqa: F811
     inst.compute_potential(1)
     assert_close(interior(inst.download("psi")), interior(o.f["psi"]), 1e-11, "psi", demean=True)
     inst.close()
+
+
+# itot at the edges of the stencil blocks (124 columns, the ux pairs one
+# column early) and of the rows' shapes (2, 4 and 8 unknowns per thread, by the
+# number of rows), odd row counts, one wave to sixteen
+ROW_CASES = [(4, 4), (5, 9), (123, 12), (124, 15), (125, 12), (126, 8), (248, 12), (249, 8),
+             (250, 8), (373, 1440), (512, 1024), (512, 2700), (1024, 16), (1025, 8), (4097, 6),
+             (8192, 4)]
+
+
+@pytest.mark.parametrize("imy", [0, 1])
+@pytest.mark.parametrize("itot,jtot", ROW_CASES)
+def test_row_predictor_edges(sns, itot, jtot, imy):
+    """Two fused steps (the corrections folded into the predictor with
+    explicit y) against the reference-named functions, whose source terms
+    equal the oracle's bit for bit: every field equal, stretched grid."""
+    if imy and jtot < 16:
+        jtot = 16
+    fields = {}
+    for fused in (False, True):
+        inst = sns.Instance(itot, jtot, stretch=3.0, Ra=1e7, Pr=2.0, implicitx=1, implicity=imy)
+        inst.alloc()
+        inst.state_alloc()
+        rng = np.random.default_rng(itot + jtot)
+        for n in ("ux", "uy", "p", "temp"):
+            inst.upload(n, 0.1 * rng.standard_normal(inst.shape(n)))
+            inst.update_boundaries(n)
+            inst.state_upload(n, inst.download(n))
+        inst.set_dt(1e-4)
+        for _ in range(2):
+            inst.integrate() if fused else inst.integrate_reference_order()
+        for n in ("ux", "uy", "p", "temp"):
+            inst.update_boundaries(n)
+            got = inst.state_download(n) if fused else inst.download(n)
+            assert np.isfinite(got).all()
+            if fused:
+                assert np.array_equal(got, fields[n]), (n, np.abs(got - fields[n]).max())
+            fields[n] = got
+        inst.close()
