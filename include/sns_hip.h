@@ -230,10 +230,10 @@ typedef struct {
   int ysolve_recompute; /* its chunk interiors: 1 solved again in the apply
                            kernel, 2 stored and read back */
   int split_corr;       /* 1: every substage ends with the correction kernel;
-                           0 (the rule): with implicit x and explicit y the
-                           predictors of substages 2 and 3 apply the previous
-                           substage's correction to the fields as they load
-                           them (the same operations, so the same bits) */
+                           0 (the rule): with explicit y the predictors of
+                           substages 2 and 3 apply the previous substage's
+                           correction to the fields as they load them (the
+                           same operations, so the same bits) */
 } snsg_launch;
 /* SNSG_E_ARG for a value outside the ranges above, SNSG_E_SIZE for one the
  * grid does not admit (a factor that does not divide jtot or whose FFT pass

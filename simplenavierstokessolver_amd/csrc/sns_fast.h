@@ -147,25 +147,11 @@ __device__ __forceinline__ double ldr(const double *row, int k) {
 __device__ __forceinline__ void str(double *row, int k, double v) {
   *reinterpret_cast<double *>(reinterpret_cast<char *>(row) + ((unsigned)k << 3)) = v;
 }
-// Rows j-1, j, j+1 of a field: pointers to the first stored element of each
-// row (I = 0 for uy, p, psi, T; I = 1 for ux).
-struct Rows3 {
-  const double *m, *c, *p;
-};
-__device__ __forceinline__ Rows3 ux_rows(const Geo &g, const double *f, int j) {
-  const size_t w = (size_t)g.pu;
-  return {f + (size_t)(j - 1) * w, f + (size_t)j * w, f + (size_t)(j + 1) * w};
-}
-__device__ __forceinline__ Rows3 c_rows(const Geo &g, const double *f, int j) {
-  const size_t w = (size_t)g.pc;
-  return {f + (size_t)(j - 1) * w, f + (size_t)j * w, f + (size_t)(j + 1) * w};
-}
 
 // ------------------------------------------------------------ source terms
 //
 // Each source term is written once, on the values around the point; the
-// loaders below (pointer form) and the row kernels (values shared across
-// lanes and rows) feed it.  Operation order follows the reference
+// predictors feed it with values shared across lanes and rows (sns_rows.h).  Operation order follows the reference
 // expression by expression.
 
 // Split of the diffusive terms dif1 (x), dif2 (y) between the explicit part
@@ -226,15 +212,6 @@ __device__ __forceinline__ void temp_src_g(const Geo &g, const Tables &tb, const
   srcg = w.g(dif1, dif2);
 }
 
-template <bool LANE = false, bool P2 = false, class W>
-__device__ __forceinline__ void temp_src_v(const Geo &g, const Tables &tb, const CellX &x,
-                                           const TempPt &v, const W &w, double &srca,
-                                           double &srcg) {
-  const double dtdx_xp = dv<P2>(-v.t_c + v.t_xp, x.dxc_p, x.rdxc_p);
-  const double dtdx_xm = LANE ? from_left(dtdx_xp) : dv<P2>(-v.t_xm + v.t_c, x.dxc, x.rdxc);
-  temp_src_g<P2>(g, tb, x, v, dtdx_xm, dtdx_xp, w, srca, srcg);
-}
-
 // x-momentum at face (i, j), i = 2..itot: src/fluid/update_velocity.c:34-101
 struct UxPt {
   double u_c, u_xm, u_xp, u_ym, u_yp;  // UX(i,j), UX(i-1,j), UX(i+1,j), UX(i,j-1), UX(i,j+1)
@@ -269,16 +246,6 @@ __device__ __forceinline__ void ux_src_g(const Geo &g, const Tables &tb, const F
   srcg = w.g(dif1, dif2) + pre;
 }
 
-template <bool LANE = false, bool P2 = false, class W>
-__device__ __forceinline__ void ux_src_v(const Geo &g, const Tables &tb, const FaceX &x,
-                                         const UxPt &v, const W &w, double &srca,
-                                         double &srcg) {
-  const double duxdx_xp = dv<P2>(-v.u_c + v.u_xp, x.dxf, x.rdxf);
-  const double duxdx_xm =
-      LANE ? from_left(duxdx_xp) : dv<P2>(-v.u_xm + v.u_c, x.dxf_m, x.rdxf_m);
-  ux_src_g<P2>(g, tb, x, v, duxdx_xm, duxdx_xp, w, srca, srcg);
-}
-
 // y-momentum at (i, j), i = 1..itot: src/fluid/update_velocity.c:128-189
 struct UyPt {
   double v_c, v_xm, v_xp, v_ym, v_yp;  // UY(i,j), UY(i-1,j), UY(i+1,j), UY(i,j-1), UY(i,j+1)
@@ -305,59 +272,6 @@ __device__ __forceinline__ void uy_src_g(const Geo &g, const Tables &tb, const C
   const double pre = dv<P2>(-(v.p_c - v.p_ym), dy, rdy);
   srca = w.a(+(adv1 + adv2), dif1, dif2);
   srcg = w.g(dif1, dif2) + pre;
-}
-
-template <bool LANE = false, bool P2 = false, class W>
-__device__ __forceinline__ void uy_src_v(const Geo &g, const Tables &tb, const CellX &x,
-                                         const UyPt &v, const W &w, double &srca,
-                                         double &srcg) {
-  const double duydx_xp = dv<P2>(-v.v_c + v.v_xp, x.dxc_p, x.rdxc_p);
-  const double duydx_xm = LANE ? from_left(duydx_xp) : dv<P2>(-v.v_xm + v.v_c, x.dxc, x.rdxc);
-  uy_src_g<P2>(g, tb, x, v, duydx_xm, duydx_xp, w, srca, srcg);
-}
-
-// ------------------------------------------------ loaders (pointer form)
-
-__device__ __forceinline__ CellX cell_x(const Tables &tb, int i) {
-  return {ldr(tb.dxc(), i - 1), ldr(tb.rdxc(), i - 1), ldr(tb.dxc(), i),   ldr(tb.rdxc(), i),
-          ldr(tb.dxf(), i - 1), ldr(tb.rdxf(), i - 1), ldr(tb.cT_xm(), i - 1), ldr(tb.cT_xp(), i - 1)};
-}
-__device__ __forceinline__ FaceX face_x(const Tables &tb, int i) {
-  return {ldr(tb.dxf(), i - 2),   ldr(tb.rdxf(), i - 2),  ldr(tb.dxf(), i - 1), ldr(tb.rdxf(), i - 1),
-          ldr(tb.cU_xm(), i - 1), ldr(tb.cU_xp(), i - 1), ldr(tb.dxc(), i - 1), ldr(tb.rdxc(), i - 1)};
-}
-
-template <bool P2 = false>
-__device__ __forceinline__ void temp_src_t(const Geo &g, const Tables &tb, const Rows3 &ux,
-                                           const Rows3 &uy, const Rows3 &temp, int i, double wex,
-                                           double wey, double wix, double wiy, double &srca,
-                                           double &srcg) {
-  const TempPt v = {ldr(temp.c, i), ldr(temp.c, i - 1), ldr(temp.c, i + 1), ldr(temp.m, i),
-                    ldr(temp.p, i), ldr(ux.c, i - 1),   ldr(ux.c, i),       ldr(uy.c, i),
-                    ldr(uy.p, i)};
-  temp_src_v<false, P2>(g, tb, cell_x(tb, i), v, Weights<>{wex, wey, wix, wiy}, srca, srcg);
-}
-
-template <bool P2 = false>
-__device__ __forceinline__ void ux_src_t(const Geo &g, const Tables &tb, const Rows3 &ux,
-                                         const Rows3 &uy, const Rows3 &p, double tf, int i,
-                                         double wex, double wey, double wix, double wiy,
-                                         double &srca, double &srcg) {
-  const UxPt v = {ldr(ux.c, i - 1), ldr(ux.c, i - 2), ldr(ux.c, i), ldr(ux.m, i - 1),
-                  ldr(ux.p, i - 1), ldr(uy.c, i - 1), ldr(uy.c, i), ldr(uy.p, i - 1),
-                  ldr(uy.p, i),     ldr(p.c, i),      ldr(p.c, i - 1), tf};
-  ux_src_v<false, P2>(g, tb, face_x(tb, i), v, Weights<>{wex, wey, wix, wiy}, srca, srcg);
-}
-
-template <bool P2 = false>
-__device__ __forceinline__ void uy_src_t(const Geo &g, const Tables &tb, const Rows3 &ux,
-                                         const Rows3 &uy, const Rows3 &p, int i, double wex,
-                                         double wey, double wix, double wiy, double &srca,
-                                         double &srcg) {
-  const UyPt v = {ldr(uy.c, i),     ldr(uy.c, i - 1), ldr(uy.c, i + 1), ldr(uy.m, i),
-                  ldr(uy.p, i),     ldr(ux.m, i - 1), ldr(ux.c, i - 1), ldr(ux.m, i),
-                  ldr(ux.c, i),     ldr(p.c, i),      ldr(p.m, i)};
-  uy_src_v<false, P2>(g, tb, cell_x(tb, i), v, Weights<>{wex, wey, wix, wiy}, srca, srcg);
 }
 
 // ---------------------------------------------------------------- stores

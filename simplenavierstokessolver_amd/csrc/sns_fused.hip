@@ -16,104 +16,123 @@
 #include "sns_launch.h"
 #include "sns_fast.h"
 #include "sns_fused.h"
-#include "sns_lu.h"
+#include "sns_rows.h"
 
 namespace sns {
 
 // ------------------------------------------------------------- predictor
 
-// Row pointers of the substage-start fields around row j (j uniform across
-// the workgroup) and of row j of the RK histories.
-struct PredRows {
-  Rows3 ux, uy, t, p;
-  double *hu, *hv, *ht;
-};
+// Explicit diffusion in x: the source terms of one field in one block of
+// columns and one pair of rows per wave (sns_rows.h), the final values with
+// boundary values, or the increments when a y solve follows (IMY).  FOLD: the
+// previous substage's correction is applied to the fields as they are loaded.
+//
+// Small grids are bound by latency (a launch, a load, a chain of divisions, a
+// store), larger ones by the loads: one thread per cell loaded 45 to 60 words
+// one at a time, 10 neighbours of each field and the column metrics.  us per
+// launch, one thread per cell and now: 700x1000 without T 19.1 and 14.3 (16.3
+// with the rows loaded one after the other and two idle waves a workgroup),
+// 128x192 5.4 and 5.2, folded 5.9 in place of 5.4 and a correction of 4.2.
+// A step of 32x64 takes 79 us instead of 87, twenty of 128x192 1.55 ms
+// instead of 1.79: two launches fewer a step.
+constexpr int kExpWaves = 4;
 
-__device__ __forceinline__ PredRows pred_rows(const PredArgs &a, int j) {
+template <int F, bool P2, bool FOLD, int IMY>
+__device__ __forceinline__ void pred_exp_body(const PredArgs &a, int b, int ja, int jb,
+                                              bool write_a) {
   const Geo &g = a.g;
-  PredRows r;
-  r.ux = ux_rows(g, a.ux, j);
-  r.uy = c_rows(g, a.uy, j);
-  r.t = c_rows(g, a.temp, j);
-  r.p = c_rows(g, a.p, j);
-  r.hu = a.hist_ux + (size_t)(j - 1) * (g.itot - 1);
-  r.hv = a.hist_uy + (size_t)(j - 1) * g.itot;
-  r.ht = a.hist_t + (size_t)(j - 1) * g.itot;
-  return r;
-}
-
-// Increment of field f (0: T, 1: ux, 2: uy) at (i, j); the RK history of the
-// explicit terms is read (beta != 0) and rewritten in place.
-template <bool P2>
-__device__ __forceinline__ double pred_field(const PredArgs &a, const PredRows &R, int f, int i,
-                                             double dt) {
-  const Geo &g = a.g;
-  double A, G, B = 0.;
-  if (f == 0) {
-    temp_src_t<P2>(g, a.tb, R.ux, R.uy, R.t, i, a.tr.w_ex_x, a.tr.w_ex_y, a.tr.w_im_x, a.tr.w_im_y,
-               A, G);
-    if (a.read_hist) B = ldr(R.ht, i - 1);
-    if (a.write_hist) str(R.ht, i - 1, A);
-  } else if (f == 1) {
-    double tf = 0.;
-    if (a.forcing) tf = 0.5 * ldr(R.t.c, i - 1) + 0.5 * ldr(R.t.c, i);
-    ux_src_t<P2>(g, a.tb, R.ux, R.uy, R.p, tf, i, a.tr.w_ex_x, a.tr.w_ex_y, a.tr.w_im_x,
-             a.tr.w_im_y, A, G);
-    if (a.read_hist) B = ldr(R.hu, i - 2);
-    if (a.write_hist) str(R.hu, i - 2, A);
-  } else {
-    uy_src_t<P2>(g, a.tb, R.ux, R.uy, R.p, i, a.tr.w_ex_x, a.tr.w_ex_y, a.tr.w_im_x, a.tr.w_im_y, A,
-             G);
-    if (a.read_hist) B = ldr(R.hv, i - 1);
-    if (a.write_hist) str(R.hv, i - 1, A);
-  }
-  return rk_incr(a.alpha, a.beta, a.gamma, dt, A, B, G);
-}
-
-// Final value of field f at (i, j), or its x-aligned increment when a y
-// solve follows.
-__device__ __forceinline__ void emit_field(const PredArgs &a, const PredRows &R, int f, int i,
-                                           int j, double d) {
-  const Geo &g = a.g;
-  if (f == 0) {
-    if (a.q_t) str(a.q_t + (size_t)(j - 1) * g.itot, i - 1, d);
-    else put_c<2>(g, a.out_t, i, j, ldr(R.t.c, i) + d);
-  } else if (f == 1) {
-    if (a.q_u) str(a.q_u + (size_t)(j - 1) * (g.itot - 1), i - 2, d);
-    else put_ux(g, a.out_u, i, j, ldr(R.ux.c, i - 1) + d);
-  } else {
-    if (a.q_v) str(a.q_v + (size_t)(j - 1) * g.itot, i - 1, d);
-    else put_c<0>(g, a.out_v, i, j, ldr(R.uy.c, i) + d);
-  }
-}
-
-// explicit diffusion in x: point-wise, the three fields per thread
-template <bool P2, class S>
-__global__ void __launch_bounds__(256) k_pred_exp(S src) {
-  const PredArgs a = src.get();
-  const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-  const int j = xcd_remap(blockIdx.y, gridDim.y) + 1;
-  if (i > a.g.itot) return;
+  const int itot = g.itot;
+  const int n = F == 1 ? itot - 1 : itot;
+  const int i0 = F == 1 ? 2 : 1;
   const double dt = *a.dtp;
-  const PredRows R = pred_rows(a, j);
-  if (a.with_temp) emit_field(a, R, 0, i, j, pred_field<P2>(a, R, 0, i, dt));
-  if (i >= 2) emit_field(a, R, 1, i, j, pred_field<P2>(a, R, 1, i, dt));
-  emit_field(a, R, 2, i, j, pred_field<P2>(a, R, 2, i, dt));
+  const LanePos p = lane_pos(1 + b * kBlockCols - 2, i0, n, itot, 0, n, 1, 63);
+  const bool edge = (F == 1 && b == 0) || (b + 1) * kBlockCols >= n;
+  const RowSrc<F, FOLD> q = row_src<F, FOLD>(a, ja, jb, n);
+  const unsigned pitch = (unsigned)(IMY ? n : F == 1 ? g.pu : g.pc) * 8u;
+  const unsigned rows = (unsigned)(IMY ? g.jtot : g.jtot + 2);
+  double *dst = IMY ? (F == 0 ? a.q_t : F == 1 ? a.q_u : a.q_v)
+                    : (F == 0 ? a.out_t : F == 1 ? a.out_u : a.out_v);
+  const Buf out = IMY || F == 1 ? buf_of(dst, pitch * rows) : cell_buf(dst, pitch * rows);
+  // result of row j at byte offset `row`; `halo`: its periodic copy's row
+  auto emit = [&](double2 d, double2 own, int j, bool copy, unsigned halo) {
+    const unsigned row = (unsigned)(IMY ? j - 1 : j) * pitch;
+    if constexpr (IMY) {
+      store_hist(out, p, edge, row, d);
+    } else {
+      const double2 v = make_double2(own.x + d.x, own.y + d.y);
+      const unsigned o = F == 1 ? p.u : p.c;
+      store_pair(out, p, edge, o, row, v);
+      if (copy) store_pair(out, p, edge, o, halo, v);
+      if (p.interior) return;
+      // wall values, by the lanes that hold the first and the last unknown
+      // (T's walls end at rows 1 and jtot)
+      const bool first = (p.out0 && p.ii == 0) || (p.out1 && p.ii + 1 == 0);
+      const bool last = (p.out0 && p.ii == n - 1) || (p.out1 && p.ii + 1 == n - 1);
+      const unsigned wl = first ? (F == 1 ? 0u : 8u) : kOff;
+      const unsigned wr = last ? (unsigned)(F == 1 ? itot : itot + 2) * 8u : kOff;
+      bst(out, wl, row, F == 0 ? +0.5 : 0.);
+      bst(out, wr, row, F == 0 ? -0.5 : 0.);
+      if (F != 0 && copy) {
+        bst(out, wl, halo, 0.);
+        bst(out, wr, halo, 0.);
+      }
+    }
+  };
+  // both rows' loads first: one wait instead of two
+  Raw<F> r;
+  double2 da, db;
+  raw_load<F, P2, FOLD, 0>(a.tb, q, p, r);
+  raw_load<F, P2, FOLD, 1>(a.tb, q, p, r);
+  if constexpr (FOLD) {
+    raw_fold<F, P2, 0, 0, 0>(a, q, p, ja, jb, write_a, edge, dt, r);
+    raw_fold<F, P2, 0, 0, 1>(a, q, p, ja, jb, write_a, edge, dt, r);
+  }
+  raw_eval<F, P2, 0, IMY, 0>(a, q, r, p, write_a, edge, dt, da);
+  raw_eval<F, P2, 0, IMY, 1>(a, q, r, p, write_a, edge, dt, db);
+  if (write_a) emit(da, r.own_a(), ja, ja == 1, (unsigned)(g.jtot + 1) * pitch);
+  emit(db, r.own_b(), jb, jb == g.jtot, 0u);
 }
 
-// Power-of-two divisors select the variant that divides by multiplying.
+// Workgroup w: blocks (w % ncg)*waves .. of field (w / ncg) % nfld (+1 without
+// the temperature equation), row pair w / ncg / nfld (as k_pred_rows).
+template <bool P2, bool FOLD, int IMY, class S>
+__global__ void __launch_bounds__(64 * kExpWaves, 3) k_pred_exp(S src, int nfld, int ncg) {
+  const PredArgs a = src.get();
+  const int w = xcd_groups(blockIdx.x, gridDim.x, kPredGroup * nfld * ncg);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int b = (w % ncg) * (blockDim.x >> 6) + wave;
+  const int r = w / ncg;
+  const int q = r / nfld, f = r % nfld + (nfld == 3 ? 0 : 1);
+  if (b * kBlockCols >= a.g.itot) return;
+  const int ja = min(2 * q + 1, a.g.jtot - 1), jb = ja + 1;
+  const bool write_a = ja == 2 * q + 1;
+  if (f == 0) pred_exp_body<0, P2, FOLD, IMY>(a, b, ja, jb, write_a);
+  else if (f == 1) pred_exp_body<1, P2, FOLD, IMY>(a, b, ja, jb, write_a);
+  else pred_exp_body<2, P2, FOLD, IMY>(a, b, ja, jb, write_a);
+}
+
+// Power-of-two divisors select the variant that divides by multiplying, a psi
+// argument the one that applies the previous substage's correction.
 template <class S>
 static void pred_exp_launch(hipStream_t s, const PredArgs &shape, S src, int nz) {
   const Geo &g = shape.g;
-  const dim3 grid((g.itot + 255) / 256, g.jtot, nz);
-  if (pow2_division(shape.tb))
-    hipLaunchKernelGGL((k_pred_exp<true, S>), grid, dim3(256), 0, s, src);
-  else
-    hipLaunchKernelGGL((k_pred_exp<false, S>), grid, dim3(256), 0, s, src);
+  const int nb = (g.itot + kBlockCols - 1) / kBlockCols;
+  const int ncg = (nb + kExpWaves - 1) / kExpWaves, waves = (nb + ncg - 1) / ncg;
+  const int nfld = shape.with_temp ? 3 : 2;
+  const dim3 grid((g.jtot + 1) / 2 * nfld * ncg, 1, nz), block(64 * waves);
+  const bool p2 = pow2_division(shape.tb), fold = shape.psi != nullptr;
+  const bool imy = shape.tr.implicity;  // excludes fold
+#define SNS_CALL(P2, FOLD, IMY) \
+  hipLaunchKernelGGL((k_pred_exp<P2, FOLD, IMY, S>), grid, block, 0, s, src, nfld, ncg)
+  if (p2 && fold) SNS_CALL(true, true, 0);
+  else if (p2 && imy) SNS_CALL(true, false, 1);
+  else if (p2) SNS_CALL(true, false, 0);
+  else if (fold) SNS_CALL(false, true, 0);
+  else if (imy) SNS_CALL(false, false, 1);
+  else SNS_CALL(false, false, 0);
+#undef SNS_CALL
 }
 
-// A folded correction (psi set) is only requested with implicit x: the
-// explicit-x kernel takes its fields as they are.
 void launch_pred(hipStream_t s, const PredArgs &a, int implicitx) {
   if (implicitx) launch_pred_rows(s, a);
   else pred_exp_launch(s, a, ArgOne<PredArgs>{a}, 1);

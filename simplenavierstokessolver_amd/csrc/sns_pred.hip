@@ -210,12 +210,9 @@ __device__ __forceinline__ int pad_idx(int r) {
   return r + (int)((unsigned)r / M);
 }
 
-// Stencil blocks: kBlockCols adjacent columns, two per lane (sns_rows.h), lanes
-// 0 and 63 holding the neighbours.  Block k of wave w is number k*NW + w of the
-// row, so the waves of a workgroup work side by side and share the cache lines
-// at the block ends while those are in L1.
-constexpr int kBlockCols = 124;
-
+// Stencil blocks of kBlockCols adjacent columns.  Block k of wave w is number
+// k*NW + w of the row, so the waves of a workgroup work side by side and share
+// the cache lines at the block ends while those are in L1.
 template <int NW>
 __device__ __forceinline__ LanePos block_pos(int k, int i0, int n, int itot) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -400,21 +397,6 @@ __device__ __forceinline__ void pred_rows_body(const PredArgs &a, PredRowsLds<NT
       if (F != 0 && (second ? copy_b : copy_a)) bst(out, wo, second ? 0u : top, wv);
     }
   }
-}
-
-// Row pairs of one XCD's run before the next XCD's (xcd_groups): rows that
-// share neighbours meet in an L2, and the eight runs stay close in memory.
-// 2048x4096 IMP-IMP, us per launch: 234 with an eighth of the grid per XCD,
-// 232, 227, 226 and 224 with 1, 4, 8 and 64 pairs, 256 without any order.
-constexpr int kPredGroup = 64;
-
-// Waves per SIMD: the two rows' LDS leaves 4 (two workgroups per CU) at the
-// widest rows; the folded kernel with the division sequence needs 156
-// registers, so on narrower rows it takes 3 (1537x3000: 206 us, 220 with 4 and
-// spilled registers).
-template <bool P2, bool FOLD, int NT>
-constexpr int pred_waves() {
-  return FOLD && !P2 && NT <= 256 ? 3 : 4;
 }
 
 // Workgroup w: field w % nfld (+1 without the temperature equation) of rows

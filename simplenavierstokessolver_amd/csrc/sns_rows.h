@@ -20,6 +20,24 @@
 
 namespace sns {
 
+// Columns of a block: two per lane, lanes 0 and 63 hold the neighbours
+constexpr int kBlockCols = 124;
+
+// Row pairs of one XCD's run before the next XCD's (xcd_groups): rows that
+// share neighbours meet in an L2, and the eight runs stay close in memory.
+// 2048x4096 IMP-IMP, us per launch: 234 with an eighth of the grid per XCD,
+// 232, 227, 226 and 224 with 1, 4, 8 and 64 pairs, 256 without any order.
+constexpr int kPredGroup = 64;
+
+// Waves per SIMD: the two rows' LDS leaves 4 (two workgroups per CU) at the
+// widest rows; the folded kernel with the division sequence needs 156
+// registers, so on narrower rows it takes 3 (1537x3000: 206 us, 220 with 4 and
+// spilled registers).
+template <bool P2, bool FOLD, int NT>
+constexpr int pred_waves() {
+  return FOLD && !P2 && NT <= 256 ? 3 : 4;
+}
+
 // Columns of a lane and their byte offsets: in rows of the cell arrays (c,
 // relative to element -1, which the rows' padding holds), of ux (u), of the
 // column tables (t) and of the RK history and increments (h).  out0, out1: the
@@ -118,18 +136,27 @@ template <int F>
 struct Raw;
 template <>
 struct Raw<0> {
+  // the field's own values, what the increments are added to
+  __device__ __forceinline__ double2 own_a() const { return t_a; }
+  __device__ __forceinline__ double2 own_b() const { return t_b; }
   double2 t_am, t_a, t_b, t_bp, u_a, u_b, v_a, v_b, v_bp, ba, bb;
   double2 s_am, s_a, s_b, s_bp;
   Metric x;
 };
 template <>
 struct Raw<1> {
+  // the field's own values, what the increments are added to
+  __device__ __forceinline__ double2 own_a() const { return u_a; }
+  __device__ __forceinline__ double2 own_b() const { return u_b; }
   double2 u_am, u_a, u_b, u_bp, v_a, v_b, v_bp, p_a, p_b, t_a, t_b, ba, bb;
   double2 s_am, s_a, s_b, s_bp;
   Metric x;
 };
 template <>
 struct Raw<2> {
+  // the field's own values, what the increments are added to
+  __device__ __forceinline__ double2 own_a() const { return v_a; }
+  __device__ __forceinline__ double2 own_b() const { return v_b; }
   double2 v_am, v_a, v_b, v_bp, u_am, u_a, u_b, p_am, p_a, p_b, ba, bb;
   double2 s_amm, s_am, s_a, s_b, s_bp;
   Metric x;

@@ -107,3 +107,43 @@ def test_row_predictor_edges(sns, itot, jtot, imy):
                 assert np.array_equal(got, fields[n]), (n, np.abs(got - fields[n]).max())
             fields[n] = got
         inst.close()
+
+
+# itot at the edges of the blocks (124 columns) and of the workgroups (four
+# blocks), odd row counts; powers of two with stretch 0 divide by multiplying
+EXP_CASES = [(4, 4, 0.), (5, 9, 3.), (64, 64, 0.), (123, 12, 3.), (124, 15, 0.), (125, 12, 3.),
+             (128, 192, 0.), (248, 9, 3.), (249, 8, 0.), (497, 12, 3.), (512, 32, 0.),
+             (1024, 15, 0.)]
+
+
+@pytest.mark.parametrize("imy", [0, 1])
+@pytest.mark.parametrize("with_t", [1, 0])
+@pytest.mark.parametrize("itot,jtot,stretch", EXP_CASES)
+def test_explicit_x_predictor_edges(sns, itot, jtot, stretch, with_t, imy):
+    """Explicit diffusion in x: two fused steps (the corrections folded into
+    the predictor with explicit y) against the reference-named functions:
+    every field equal."""
+    if imy and jtot < 16:
+        jtot = 16
+    fields = {}
+    for fused in (False, True):
+        inst = sns.Instance(itot, jtot, stretch=stretch, Ra=1e7, Pr=2.0, implicitx=0,
+                            implicity=imy, with_temperature=with_t)
+        inst.alloc()
+        inst.state_alloc()
+        rng = np.random.default_rng(itot + jtot)
+        for n in ("ux", "uy", "p", "temp"):
+            inst.upload(n, 0.1 * rng.standard_normal(inst.shape(n)))
+            inst.update_boundaries(n)
+            inst.state_upload(n, inst.download(n))
+        inst.set_dt(1e-6)
+        for _ in range(2):
+            inst.integrate() if fused else inst.integrate_reference_order()
+        for n in ("ux", "uy", "p", "temp"):
+            inst.update_boundaries(n)
+            got = inst.state_download(n) if fused else inst.download(n)
+            assert np.isfinite(got).all()
+            if fused:
+                assert np.array_equal(got, fields[n]), (n, np.abs(got - fields[n]).max())
+            fields[n] = got
+        inst.close()
