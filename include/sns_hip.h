@@ -218,7 +218,9 @@ int snsg_memory(const snsg_ctx *ctx, size_t *bytes);
  * batched or served (a batch's shape classes include the shapes). */
 typedef struct {
   int fft_n1;           /* length of the first factor of the four-step y FFT
-                           (a divisor of jtot; jtot/fft_n1 the second) */
+                           (a divisor of jtot; jtot/fft_n1 the second).  In
+                           effect 0: whole columns in one kernel, which the
+                           rule takes up to 1024 rows */
   int ysolve_chunk;     /* rows per chunk of the partitioned CN-y solve: a
                            divisor of jtot in 4..32, with 4..513 chunks;
                            1: no partition (column solves on the transposed

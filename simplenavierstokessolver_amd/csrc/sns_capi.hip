@@ -334,7 +334,7 @@ extern "C" int snsg_create(int device, const snsg_config *cfg, const double *dxf
       {(void **)&c->d_eigen, sizeof(double) * (jtot / 2 + 1)},
       {(void **)&c->d_tw, sizeof(double2) * jtot},
       {(void **)&c->d_psihat, sizeof(double2) * (size_t)itot * (jtot / 2 + 1)},
-      {(void **)&c->d_Y, sizeof(double2) * (size_t)pl.npair * jtot},
+      {(void **)&c->d_Y, sizeof(double2) * fft2_work(pl)},
       {(void **)&c->d_q, sizeof(double) * (size_t)(itot + 1) * jtot},
       {(void **)&c->d_qy, sizeof(double) * (size_t)(itot + 1) * jtot},
       {(void **)&c->d_red, sizeof(unsigned long long)},
@@ -400,7 +400,7 @@ snsg_launch tuned_launch(int itot, int jtot) {
 LaunchKey launch_key(int itot, int jtot, const snsg_launch &req) {
   LaunchKey k{};
   Fft2Plan pl;
-  k.n1 = fft2_plan(jtot, itot, pl, req.fft_n1) ? pl.n1 : 0;
+  k.n1 = fft2_plan(jtot, itot, pl, req.fft_n1) && !pl.one ? pl.n1 : 0;
   // chunk 1: the column solves on the transposed increments (also where
   // jtot has no chunk length the partitioned solve takes)
   k.chunk = req.ysolve_chunk ? req.ysolve_chunk : ysolve_chunk(jtot);
@@ -420,7 +420,7 @@ LaunchKey launch_key(int itot, int jtot, const snsg_launch &req) {
 
 LaunchKey launch_key(const snsg_ctx *c) {
   LaunchKey k = launch_key(c->geo.itot, c->geo.jtot, c->launch);
-  k.n1 = c->plan.n1;
+  k.n1 = c->plan.one ? 0 : c->plan.n1;
   return k;
 }
 
@@ -898,7 +898,7 @@ extern "C" int snsg_instance_bytes(const snsg_config *cfg, size_t *bytes) {
   size_t n = 0;
   // snsg_create
   n += d * itot + d * (itot + 1) + d + d + d * (jtot / 2 + 1) + z * jtot;
-  n += z * itot * (jtot / 2 + 1) + z * (size_t)pl.npair * jtot;
+  n += z * itot * (jtot / 2 + 1) + z * fft2_work(pl);
   n += 2 * d * (itot + 1) * jtot + sizeof(unsigned long long);
   n += d * kTables * stride + z * kTables2 * stride;
   n += d * poisson_factor_doubles((int)itot, (int)jtot) + d * 2 * (size_t)poisson_factor_entries((int)itot);

@@ -36,7 +36,7 @@ struct snsg_ctx {
   Fft2Plan plan{};
   snsg_launch launch{};  // requested launch shapes (0: the rule)
   int in_batch = 0;      // batches that hold this instance
-  double2 *d_Y = nullptr;  // four-step FFT intermediate, jtot rows of (itot+1)/2 pairs
+  double2 *d_Y = nullptr;  // four-step FFT intermediate, fft2_work entries
   // per-column tables of the fused kernels (one allocation)
   double *d_tab = nullptr;
   double2 *d_tab2 = nullptr;           // paired column tables

@@ -2,21 +2,30 @@
 #pragma once
 #include "sns_launch.h"
 #include "sns_fast.h"
+#include "sns_fft.h"
 
 namespace sns {
 
+// Transforms of length n = jtot along y.  Two passes: the four-step plan
+// n = n1*n2 (s1, s2 the stages of the factors; 2^lgt column pairs and G rows
+// j2 per workgroup in passes A and A', 8 pairs in B and B').  one: whole
+// columns, 2^lgt pairs per workgroup, s1 the stages of n.
 struct Fft2Plan {
-  int n;                         // transform length (jtot) = n1*n2
+  int n;
   int n1, n2;
-  int np1, np2;                  // radix passes of the two factors
-  unsigned long long code1, code2;
-  int npair;                     // complex column pairs, (itot+1)/2
-  int G;                         // rows j2 per workgroup in passes A and A'
+  FftSched s1, s2;
+  int npair;  // complex column pairs, (itot+1)/2
+  int lgt;
+  int G;
+  bool one;
 };
 
-// four-step plan of length n for itot columns; n1 > 0 fixes the first
-// factor (false when the factors or the LDS tiles do not fit)
+// plan of length n for itot columns; n1 > 0 takes the two passes with this
+// first factor (false when the factors or the LDS tiles do not fit)
 bool fft2_plan(int n, int itot, Fft2Plan &pl, int n1 = 0);
+
+// Entries of the two passes' intermediate (whole tiles of 8 pairs)
+inline size_t fft2_work(const Fft2Plan &pl) { return (size_t)(pl.npair + 15) / 16 * 16 * pl.n; }
 
 // Thomas factors of the x systems of all wavenumbers (once per instance):
 // fac holds (jtot/2+1) tables of poisson_factor_entries(itot) reciprocal

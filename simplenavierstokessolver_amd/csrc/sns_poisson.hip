@@ -4,8 +4,8 @@
 // real FFT along y (FFTW r2c, unnormalised), one tri-diagonal system along x
 // per wavenumber, inverse c2r FFT, psi = result / jtot with Neumann walls.
 //
-// The y transforms run as four-step FFTs, n = n1*n2, j = n2*j1 + j2,
-// k = k1 + n1*k2:
+// Up to 1024 rows the y transforms take one kernel each (sns_poisson_one.hip).
+// Above, they run as four-step FFTs, n = n1*n2, j = n2*j1 + j2, k = k1 + n1*k2:
 //   forward  pass A : Y[k1*n2+j2] = W_n^(j2 k1) * DFT_n1 over j1 of x[n2 j1 + j2]
 //            pass B : X[k1 + n1 k2] = DFT_n2 over j2 of Y[k1*n2+j2]
 //   inverse  pass B': Y[k1*n2+j2] = W_n^(-j2 k1) * IDFT_n2 over k2 of Z[k1 + n1 k2]
@@ -15,287 +15,186 @@
 // columns are packed as one complex sequence, and the spectra of the pair are
 // separated (forward) or combined (inverse) in pass B / B', which therefore
 // handles the wavenumber rows k1 and n1-k1 together.
+//
+// The passes move 3, 2, 2 and 2 words per cell; from 4096x8192 (4.1, 4.8, 3.8
+// and 4.6 TB/s) they are bound by memory, whose rate the short strided runs
+// keep under that of a copy; smaller grids by a workgroup's chain of latencies.
+// us of the four passes with every stage through LDS, and with the first and
+// last stage in registers and Y in one run per tile: 1537x3000 129 and 108,
+// 1024x2048 50 and 44, 2048x4096 143 and 134, 4096x8192 570 and 562.
 #include <float.h>
 #include "sns_launch.h"
 #include "sns_fast.h"
-#include "sns_fft.h"
-#include "sns_poisson.h"
+#include "sns_poisson_dev.h"
 #include "sns_lu.h"
 
 namespace sns {
 
-static constexpr int TILE = 8;   // complex pairs per tile (16 real columns)
-static constexpr int NTF = 512;  // threads of the FFT passes
-static constexpr int EMAXF = 4;  // complex values per thread and pass
-
-// P2: every divisor a power of two (the quotients are products, see dv)
-template <bool P2>
-__device__ __forceinline__ double poisson_rhs2(const Geo &g, const Tables &tb, const double *ux,
-                                               const double *uy, double inv_gdt, int i, int j) {
-  // 1./(gamma*dt)*((ux_xp-ux_xm)/DXF(i) + (uy_yp-uy_ym)/dy)
-  const double ax = dv<P2>(ux[ux_idx(g, i + 1, j)] - ux[ux_idx(g, i, j)], tb.dxf()[i - 1],
-                           tb.rdxf()[i - 1]);
-  const double ay = dv<P2>(uy[c_idx(g, i, j + 1)] - uy[c_idx(g, i, j)], tb.dy, tb.rdy);
-  return inv_gdt * (+ax + ay);
-}
-
-__device__ __forceinline__ void put_psi(const Geo &g, double *f, int i, int j, double v) {
-  // Neumann walls and periodic halo rows (src/fluid/boundary_conditions.c:39-55)
-  f[c_idx(g, i, j)] = v;
-  if (j == 1) f[c_idx(g, i, g.jtot + 1)] = v;
-  if (j == g.jtot) f[c_idx(g, i, 0)] = v;
-  if (i == 1 || i == g.itot) {
-    const int iw = i == 1 ? 0 : g.itot + 1;
-    f[c_idx(g, iw, j)] = v;
-    if (j == 1) f[c_idx(g, iw, g.jtot + 1)] = v;
-    if (j == g.jtot) f[c_idx(g, iw, 0)] = v;
-  }
+// Intermediate of the two passes: one tile of column pairs after the other, so
+// that a workgroup of either pass stays within one run of n*128 bytes.  (Runs
+// that start off a multiple of 256 bytes cost a quarter more at 4096x8192.)
+__device__ __forceinline__ unsigned y_idx(const Fft2Plan &pl, int k1, int j2, int pair) {
+  const int t = pair >> pl.lgt, q = pair - (t << pl.lgt);
+  return (((unsigned)(t * pl.n1 + k1) * pl.n2 + j2) << pl.lgt) + q;
 }
 
 // ------------------------------------------------------------ forward A
 
-// RHS of the column pair (ia, ia+1), ia odd, at 0-based row j in 16-byte
-// loads: ux faces ia, ia+1 (one pair), ia+2; uy of rows j+1 and j+2 (one
-// pair each).  Needs the padded state layout (ux rows and uy's column 1 on
-// 16-byte boundaries, even pitches); columns past itot give 0.
-template <bool P2>
-__device__ __forceinline__ double2 poisson_rhs_pair(const Geo &g, const Tables &tb,
-                                                    const double *ux, const double *uy,
-                                                    double inv_gdt, int ia, int j) {
-  const int itot = g.itot;
-  const int ic = ia <= itot ? ia : 1;  // lanes past the last column read column 1
-  const double *urow = ux + (size_t)(j + 1) * g.pu;
-  const double2 u01 = ldr2(reinterpret_cast<const double2 *>(urow + ic - 1), 0);
-  const double u2 = ldr(urow, min(ic + 1, itot));  // face ic+2 (only used when ic+1 <= itot)
-  const double2 v0 = ldr2(reinterpret_cast<const double2 *>(uy + (size_t)(j + 1) * g.pc + ic), 0);
-  const double2 v1 = ldr2(reinterpret_cast<const double2 *>(uy + (size_t)(j + 2) * g.pc + ic), 0);
-  double dxa, rdxa, dxb, rdxb;
-  if (tb.uniform) {
-    dxa = dxb = tb.u_dxf;
-    rdxa = rdxb = tb.u_rdxf;
-  } else {
-    dxa = tb.dxf()[ic - 1];
-    rdxa = tb.rdxf()[ic - 1];
-    dxb = tb.dxf()[min(ic, itot - 1)];
-    rdxb = tb.rdxf()[min(ic, itot - 1)];
-  }
-  // the expressions of poisson_rhs2, column by column
-  const double axa = dv<P2>(u01.y - u01.x, dxa, rdxa);
-  const double aya = dv<P2>(v1.x - v0.x, tb.dy, tb.rdy);
-  const double axb = dv<P2>(u2 - u01.y, dxb, rdxb);
-  const double ayb = dv<P2>(v1.y - v0.y, tb.dy, tb.rdy);
-  double2 z;
-  z.x = ia <= itot ? inv_gdt * (+axa + aya) : 0.;
-  z.y = ia + 1 <= itot ? inv_gdt * (+axb + ayb) : 0.;
-  return z;
-}
-
-template <int L, bool P2, bool AL>
-__device__ __forceinline__ void pfwd_a(const Geo &g, const Tables &tb, const Fft2Plan &pl,
-                                       double gamma, const double *__restrict__ dtp,
-                                       const double *__restrict__ ux,
-                                       const double *__restrict__ uy,
-                                       const double2 *__restrict__ tw, double2 *__restrict__ Y) {
-  __shared__ double2 buf[EMAXF * NTF];
+template <class Sc, bool P2, bool AL>
+__device__ __forceinline__ void pfwd_a(const PoisArgs &a) {
+  extern __shared__ double2 lds_fft[];
+  const Fft2Plan &pl = a.pl;
+  const FftSched &sc = Sc::get(pl.s1);
   // consecutive tiles of one row group on the same XCD: a tile's last ux
   // face is the first of the next tile's 128-byte line, which then stays in
   // that XCD's L2
   const int nb = gridDim.x * gridDim.y;
   const int w = xcd_remap(blockIdx.y * gridDim.x + blockIdx.x, nb);
   const int tile = w % gridDim.x, j20 = (w / gridDim.x) * pl.G;
-  const int S = pl.G * TILE, n1 = pl.n1, n2 = pl.n2;
-  const FastDiv fS(S);
-  const double inv_gdt = 1. / (gamma * (*dtp));
-  for (int e = threadIdx.x; e < S * n1; e += NTF) {
-    const int j1 = fS.div(e), s = e - j1 * S;
-    const int gg = s / TILE, q = s - gg * TILE;
-    const int j = n2 * j1 + j20 + gg;  // 0-based row
-    const int ia = 2 * (tile * TILE + q) + 1;
-    double2 z;
-    if constexpr (AL) {
-      z = poisson_rhs_pair<P2>(g, tb, ux, uy, inv_gdt, ia, j);
-    } else {
-      z.x = ia <= g.itot ? poisson_rhs2<P2>(g, tb, ux, uy, inv_gdt, ia, j + 1) : 0.;
-      z.y = ia + 1 <= g.itot ? poisson_rhs2<P2>(g, tb, ux, uy, inv_gdt, ia + 1, j + 1) : 0.;
-    }
-    buf[e] = z;
-  }
-  __syncthreads();
-  if constexpr (L > 0) fft_p2<NTF, EMAXF, L, -1>(buf, __builtin_ctz(S), tw, pl.n / L);
-  else fft_il<NTF, EMAXF, -1>(buf, S, n1, pl.np1, pl.code1, tw, pl.n / n1);
-  for (int e = threadIdx.x; e < S * n1; e += NTF) {
-    const int k1 = fS.div(e), s = e - k1 * S;
-    const int gg = s / TILE, q = s - gg * TILE;
-    const int j2 = j20 + gg;
-    const int pair = tile * TILE + q;
-    if (pair < pl.npair) {
-      double2 z = buf[e];
-      if (k1 && j2) z = cmul(z, tw[j2 * k1]);
-      Y[(size_t)(k1 * n2 + j2) * pl.npair + pair] = z;
-    }
-  }
+  const int lt = pl.lgt, n2 = pl.n2;
+  const double inv_gdt = 1. / (a.gamma * (*a.dtp));
+  const FftLds l = fft_lds(lds_fft, sc, pl.G << lt, a.tw, pl.n);
+  const int pair0 = tile << lt, qm = (1 << lt) - 1;
+  fft_run<Sc, -1, true, true, AL>(
+      l, sc,
+      [&](int s) {
+        const RhsCol<P2, AL> rhs(a, inv_gdt, pair0 + (s & qm));
+        const int j2 = j20 + (s >> lt);
+        return [=](int j1) { return rhs(n2 * j1 + j2); };
+      },
+      [&](int s) {
+        const int j2 = j20 + (s >> lt), pair = pair0 + (s & qm);
+        return [=, &a](int k1, double2 z) {
+          if (pair >= a.pl.npair) return;
+          if (k1 && j2) z = cmul(z, a.tw[j2 * k1]);
+          a.Y[y_idx(a.pl, k1, j2, pair)] = z;
+        };
+      });
 }
 
 // ------------------------------------------------------------ forward B
 
-template <int L>
-__device__ __forceinline__ void pfwd_b(const Geo &g, const Fft2Plan &pl,
-                                       const double2 *__restrict__ tw,
-                                       const double2 *__restrict__ Y,
-                                       double2 *__restrict__ psihat) {
-  __shared__ double2 buf[EMAXF * NTF];
-  const int tile = blockIdx.x;
-  const int n1 = pl.n1, n2 = pl.n2, n = pl.n;
-  const int k1a = blockIdx.y, k1b = (n1 - k1a) % n1;
-  const int nh = (k1a == k1b) ? 1 : 2;
-  const int S = nh * TILE;
-  const FastDiv fS(S);
-  for (int e = threadIdx.x; e < S * n2; e += NTF) {
-    const int j2 = fS.div(e), s = e - j2 * S;
-    const int h = s / TILE, q = s - h * TILE;
-    const int pair = tile * TILE + q;
-    const int k1 = h ? k1b : k1a;
-    buf[e] = pair < pl.npair ? Y[(size_t)(k1 * n2 + j2) * pl.npair + pair] : make_double2(0., 0.);
+// The wavenumber rows k1a and k1b = n1-k1a of one tile: sequences (h << lgt) + q.
+struct PassB {
+  int pair0, k1a, k1b, nh, S;
+  int lt, qm;
+  int c0, cn;  // wavenumbers k <= n/2 of row k1a, of both
+  // the i-th of them: wavenumber and element
+  __device__ __forceinline__ int k_of(int n1, int i, int &k2, int &h) const {
+    h = i >= c0;
+    k2 = h ? i - c0 : i;
+    return (h ? k1b : k1a) + n1 * k2;
   }
-  __syncthreads();
-  if constexpr (L > 0) fft_p2<NTF, EMAXF, L, -1>(buf, __builtin_ctz(S), tw, n / L);
-  else fft_il<NTF, EMAXF, -1>(buf, S, n2, pl.np2, pl.code2, tw, n / n2);
-  // separate the two real columns of each pair: X_a = (Z_k + conj Z_{n-k})/2,
-  // X_b = (Z_k - conj Z_{n-k})/(2i), for the wavenumbers k <= n/2 of this group
-  for (int e = threadIdx.x; e < S * n2; e += NTF) {
-    const int k2 = fS.div(e), s = e - k2 * S;
-    const int h = s / TILE, q = s - h * TILE;
-    const int k1 = h ? k1b : k1a;
-    const int k = k1 + n1 * k2;
-    if (2 * k > n) continue;
-    // partner n-k = k1' + n1*k2'
-    int k2p, hp;
-    if (k1 == 0) {
-      k2p = (n2 - k2) % n2;
+  // element and sequence half of the mirror n-k of k = k1 + n1*k2
+  __device__ __forceinline__ void mirror(int n2, int k2, int h, int &k2p, int &hp) const {
+    if ((h ? k1b : k1a) == 0) {
+      k2p = k2 ? n2 - k2 : 0;
       hp = h;
     } else {
       k2p = n2 - 1 - k2;
       hp = nh == 1 ? h : 1 - h;
     }
-    const double2 zk = buf[e];
-    const double2 zn = buf[k2p * S + hp * TILE + q];
-    const int pair = tile * TILE + q;
-    const int ia = 2 * pair + 1;
-    double2 xa, xb;
-    xa.x = 0.5 * (zk.x + zn.x);
-    xa.y = 0.5 * (zk.y - zn.y);
-    xb.x = 0.5 * (zk.y + zn.y);
-    xb.y = 0.5 * (zn.x - zk.x);
-    if (ia <= g.itot) psihat[(size_t)k * g.itot + (ia - 1)] = xa;
-    if (ia + 1 <= g.itot) psihat[(size_t)k * g.itot + ia] = xb;
+  }
+};
+__device__ __forceinline__ PassB pass_b(const Fft2Plan &pl) {
+  PassB b;
+  b.lt = pl.lgt;
+  b.qm = (1 << pl.lgt) - 1;
+  b.pair0 = blockIdx.x << pl.lgt;
+  b.k1a = blockIdx.y;
+  b.k1b = b.k1a ? pl.n1 - b.k1a : 0;
+  b.nh = b.k1a == b.k1b ? 1 : 2;
+  b.S = b.nh << pl.lgt;
+  b.c0 = (pl.n / 2 - b.k1a) / pl.n1 + 1;
+  b.cn = b.c0 + (b.nh == 2 ? (pl.n / 2 - b.k1b) / pl.n1 + 1 : 0);
+  return b;
+}
+
+template <class Sc>
+__device__ __forceinline__ void pfwd_b(const PoisArgs &a) {
+  extern __shared__ double2 lds_fft[];
+  const Fft2Plan &pl = a.pl;
+  const FftSched &sc = Sc::get(pl.s2);
+  const PassB B = pass_b(pl);
+  const int n1 = pl.n1, n2 = pl.n2, n = pl.n;
+  const FftLds l = fft_lds(lds_fft, sc, B.S, a.tw, n);
+  fft_run<Sc, -1, true, false>(
+      l, sc,
+      [&](int s) {
+        const int pair = min(B.pair0 + (s & B.qm), pl.npair - 1);
+        const int k1 = s >> B.lt ? B.k1b : B.k1a;
+        return [=, &a](int j2) { return a.Y[y_idx(a.pl, k1, j2, pair)]; };
+      },
+      NoIo{});
+#pragma unroll 4
+  for (int e = threadIdx.x; e < B.cn << B.lt; e += blockDim.x) {
+    const int q = e & B.qm;
+    int k2, h, k2p, hp;
+    const int k = B.k_of(n1, e >> B.lt, k2, h);
+    B.mirror(n2, k2, h, k2p, hp);
+    put_spectra(a, k, B.pair0 + q, l.buf[fft_pad(k2 * B.S + (h << B.lt) + q)],
+                l.buf[fft_pad(k2p * B.S + (hp << B.lt) + q)]);
   }
 }
 
 // ------------------------------------------------------------ inverse B'
 
-template <int L>
-__device__ __forceinline__ void pinv_b(const Geo &g, const Fft2Plan &pl,
-                                       const double2 *__restrict__ tw,
-                                       const double2 *__restrict__ psihat,
-                                       double2 *__restrict__ Y) {
-  __shared__ double2 buf[EMAXF * NTF];
-  const int tile = blockIdx.x;
+// Each stored wavenumber m <= n/2 is read once and fills the slots of k = m
+// and of its mirror n-m, which this workgroup holds too.
+template <class Sc>
+__device__ __forceinline__ void pinv_b(const PoisArgs &a) {
+  extern __shared__ double2 lds_fft[];
+  const Fft2Plan &pl = a.pl;
+  const FftSched &sc = Sc::get(pl.s2);
+  const PassB B = pass_b(pl);
   const int n1 = pl.n1, n2 = pl.n2, n = pl.n;
-  const int k1a = blockIdx.y, k1b = (n1 - k1a) % n1;
-  const int nh = (k1a == k1b) ? 1 : 2;
-  const int S = nh * TILE;
-  const FastDiv fS(S);
-  // Hermitian extension of the two real columns' spectra packed as
-  // Z_k = X_a,k + i X_b,k (src/fluid/compute_potential.c:147-149: c2r input).
-  // Each stored wavenumber m <= n/2 is read once and fills the slots of k = m
-  // and of its mirror n-m, which this workgroup holds too (row k1 pairs with
-  // row n1-k1; the partner index is the one pass B separates with).
-  for (int e = threadIdx.x; e < S * n2; e += NTF) {
-    const int k2 = fS.div(e), s = e - k2 * S;
-    const int h = s / TILE, q = s - h * TILE;
-    const int k1 = h ? k1b : k1a;
-    const int k = k1 + n1 * k2;
-    if (2 * k > n) continue;  // filled from its mirror
-    const int pair = tile * TILE + q;
-    const int ia = 2 * pair + 1;
-    double2 xa = make_double2(0., 0.), xb = make_double2(0., 0.);
-    if (ia <= g.itot) xa = psihat[(size_t)k * g.itot + (ia - 1)];
-    if (ia + 1 <= g.itot) xb = psihat[(size_t)k * g.itot + ia];
-    if (k == 0 || 2 * k == n) { xa.y = 0.; xb.y = 0.; }
-    buf[e] = make_double2(xa.x - xb.y, xa.y + xb.x);
+  const FftLds l = fft_lds(lds_fft, sc, B.S, a.tw, n);
+#pragma unroll 4
+  for (int e = threadIdx.x; e < B.cn << B.lt; e += blockDim.x) {
+    const int q = e & B.qm;
+    int k2, h;
+    const int k = B.k_of(n1, e >> B.lt, k2, h);
+    double2 zn;
+    l.buf[fft_pad(k2 * B.S + (h << B.lt) + q)] = get_spectra(a, k, B.pair0 + q, zn);
     if (k != 0 && 2 * k != n) {
       int k2p, hp;
-      if (k1 == 0) {
-        k2p = (n2 - k2) % n2;
-        hp = h;
-      } else {
-        k2p = n2 - 1 - k2;
-        hp = nh == 1 ? h : 1 - h;
-      }
-      buf[k2p * S + hp * TILE + q] = make_double2(xa.x + xb.y, -xa.y + xb.x);
+      B.mirror(n2, k2, h, k2p, hp);
+      l.buf[fft_pad(k2p * B.S + (hp << B.lt) + q)] = zn;
     }
   }
   __syncthreads();
-  if constexpr (L > 0) fft_p2<NTF, EMAXF, L, +1>(buf, __builtin_ctz(S), tw, n / L);
-  else fft_il<NTF, EMAXF, +1>(buf, S, n2, pl.np2, pl.code2, tw, n / n2);
-  for (int e = threadIdx.x; e < S * n2; e += NTF) {
-    const int j2 = fS.div(e), s = e - j2 * S;
-    const int h = s / TILE, q = s - h * TILE;
-    const int k1 = h ? k1b : k1a;
-    const int pair = tile * TILE + q;
-    if (pair < pl.npair) {
-      double2 z = buf[e];
-      if (k1 && j2) {
-        double2 w = tw[j2 * k1];
-        w.y = -w.y;
-        z = cmul(z, w);
-      }
-      Y[(size_t)(k1 * n2 + j2) * pl.npair + pair] = z;
-    }
-  }
+  fft_run<Sc, +1, false, true>(l, sc, NoIo{}, [&](int s) {
+    const int pair = B.pair0 + (s & B.qm);
+    const int k1 = s >> B.lt ? B.k1b : B.k1a;
+    return [=, &a](int j2, double2 z) {
+      if (pair >= a.pl.npair) return;
+      if (k1 && j2) z = cmul(z, cdir<+1>(a.tw[j2 * k1]));
+      a.Y[y_idx(a.pl, k1, j2, pair)] = z;
+    };
+  });
 }
 
 // ------------------------------------------------------------ inverse A'
 
-template <int L, bool AL>
-__device__ __forceinline__ void pinv_a(const Geo &g, const Fft2Plan &pl,
-                                       const double2 *__restrict__ tw,
-                                       const double2 *__restrict__ Y, double *__restrict__ psi) {
-  __shared__ double2 buf[EMAXF * NTF];
-  const int tile = blockIdx.x, j20 = blockIdx.y * pl.G;
-  const int S = pl.G * TILE, n1 = pl.n1, n2 = pl.n2;
-  const FastDiv fS(S);
-  for (int e = threadIdx.x; e < S * n1; e += NTF) {
-    const int k1 = fS.div(e), s = e - k1 * S;
-    const int gg = s / TILE, q = s - gg * TILE;
-    const int pair = tile * TILE + q;
-    buf[e] = pair < pl.npair ? Y[(size_t)(k1 * n2 + j20 + gg) * pl.npair + pair]
-                             : make_double2(0., 0.);
-  }
-  __syncthreads();
-  if constexpr (L > 0) fft_p2<NTF, EMAXF, L, +1>(buf, __builtin_ctz(S), tw, pl.n / L);
-  else fft_il<NTF, EMAXF, +1>(buf, S, n1, pl.np1, pl.code1, tw, pl.n / n1);
-  // psi = q/jtot: the exact division of div_cr, or (jtot a power of two) the
-  // product with the exact reciprocal; both equal IEEE q/jtot bit for bit
-  const double njtot = 1. * g.jtot, rnj = 1. / njtot;
-  const bool jp2 = (g.jtot & (g.jtot - 1)) == 0;
-  for (int e = threadIdx.x; e < S * n1; e += NTF) {
-    const int j1 = fS.div(e), s = e - j1 * S;
-    const int gg = s / TILE, q = s - gg * TILE;
-    const int j = n2 * j1 + j20 + gg + 1;  // 1-based row
-    const int ia = 2 * (tile * TILE + q) + 1;
-    const double2 z = buf[e];
-    const double va = jp2 ? z.x * rnj : div_cr(z.x, njtot, rnj);
-    const double vb = jp2 ? z.y * rnj : div_cr(z.y, njtot, rnj);
-    const bool edge = j == 1 || j == g.jtot || ia == 1 || ia + 1 >= g.itot;
-    if (AL && !edge) {
-      // both columns in one 16-byte store (no halo or wall copies here)
-      *reinterpret_cast<double2 *>(psi + c_idx(g, ia, j)) = make_double2(va, vb);
-    } else {
-      if (ia <= g.itot) put_psi(g, psi, ia, j, va);
-      if (ia + 1 <= g.itot) put_psi(g, psi, ia + 1, j, vb);
-    }
-  }
+template <class Sc, bool AL>
+__device__ __forceinline__ void pinv_a(const PoisArgs &a) {
+  extern __shared__ double2 lds_fft[];
+  const Fft2Plan &pl = a.pl;
+  const FftSched &sc = Sc::get(pl.s1);
+  const int lt = pl.lgt, n2 = pl.n2, j20 = blockIdx.y * pl.G;
+  const FftLds l = fft_lds(lds_fft, sc, pl.G << lt, a.tw, pl.n);
+  const int pair0 = blockIdx.x << lt, qm = (1 << lt) - 1;
+  fft_run<Sc, +1, true, true>(
+      l, sc,
+      [&](int s) {
+        const int pair = min(pair0 + (s & qm), pl.npair - 1), j2 = j20 + (s >> lt);
+        return [=, &a](int k1) { return a.Y[y_idx(a.pl, k1, j2, pair)]; };
+      },
+      [&](int s) {
+        const PsiCol<AL> psi(a, pair0 + (s & qm));
+        const int j2 = j20 + (s >> lt);
+        return [=](int j1, double2 z) { psi(n2 * j1 + j2, z); };
+      });
 }
 
 // --------------------------------------------------- x solve per wavenumber
@@ -412,54 +311,18 @@ __device__ __forceinline__ void poisson_x3(const Geo &g, const Tables &tb,
 // Argument source S: ArgOne<PoisArgs> (one instance) or ArgBatch<PoisArgs>
 // (instance blockIdx.z of a batch).
 
-template <int L, class S>
-__global__ void __launch_bounds__(NTF) k_pfwd_a(S src) {
-  const PoisArgs a = src.get();
-  pfwd_a<L, false, false>(a.g, a.tb, a.pl, a.gamma, a.dtp, a.ux, a.uy, a.tw, a.Y);
-}
-
-// the same on the padded state layout (pair loads), with the division
-// sequence or, P2, with power-of-two divisors
-template <int L, class S>
-__global__ void __launch_bounds__(NTF) k_pfwd_a_al(S src) {
-  const PoisArgs a = src.get();
-  pfwd_a<L, false, true>(a.g, a.tb, a.pl, a.gamma, a.dtp, a.ux, a.uy, a.tw, a.Y);
-}
-template <int L, class S>
-__global__ void __launch_bounds__(NTF) k_pfwd_a_p2(S src) {
-  const PoisArgs a = src.get();
-  pfwd_a<L, true, true>(a.g, a.tb, a.pl, a.gamma, a.dtp, a.ux, a.uy, a.tw, a.Y);
-}
-
-template <int L, class S>
-__global__ void __launch_bounds__(NTF, 8) k_pfwd_b(S src) {
-  const PoisArgs a = src.get();
-  pfwd_b<L>(a.g, a.pl, a.tw, a.Y, a.psihat);
-}
+// Forward: AL on the padded state layout (pair loads), P2 with power-of-two
+// divisors; inverse: AL on the padded state layout (psi's column 1 on a
+// 16-byte boundary).
+SNS_FFT_KERNEL(pfwd_a, bool P2 SNS_C bool AL SNS_C, SNS_C P2 SNS_C AL)
+SNS_FFT_KERNEL(pfwd_b, , )
+SNS_FFT_KERNEL(pinv_b, , )
+SNS_FFT_KERNEL(pinv_a, bool AL SNS_C, SNS_C AL)
 
 template <int NT, int M, class S>
 __global__ void __launch_bounds__(NT) k_poisson_x3(S src) {
   const PoisArgs a = src.get();
   poisson_x3<NT, M>(a.g, a.tb, a.fac, a.plu, NT * M, a.psihat);
-}
-
-template <int L, class S>
-__global__ void __launch_bounds__(NTF) k_pinv_b(S src) {
-  const PoisArgs a = src.get();
-  pinv_b<L>(a.g, a.pl, a.tw, a.psihat, a.Y);
-}
-
-// the same on the padded state layout (psi's column 1 on a 16-byte boundary)
-template <int L, class S>
-__global__ void __launch_bounds__(NTF, 8) k_pinv_a_al(S src) {
-  const PoisArgs a = src.get();
-  pinv_a<L, true>(a.g, a.pl, a.tw, a.Y, a.psi);
-}
-
-template <int L, class S>
-__global__ void __launch_bounds__(NTF, 8) k_pinv_a(S src) {
-  const PoisArgs a = src.get();
-  pinv_a<L, false>(a.g, a.pl, a.tw, a.Y, a.psi);
 }
 
 // Threads NT and unknowns per thread M of the x solve for n = itot unknowns
@@ -514,97 +377,121 @@ static void px_launch(hipStream_t s, const Geo &g, S src, int nz) {
 
 // ------------------------------------------------------------- plan, launch
 
-static bool radix_code(int m, int &np, unsigned long long &code) {
-  int rest = m;
-  np = 0;
-  code = 0;
-  auto push = [&](int r) {
-    code |= (unsigned long long)r << (4 * np);
-    np++;
-    rest /= r;
-  };
-  while (rest % 8 == 0 && np < 16) push(8);
-  while (rest % 4 == 0 && np < 16) push(4);
-  while (rest % 2 == 0 && np < 16) push(2);
-  while (rest % 3 == 0 && np < 16) push(3);
-  while (rest % 5 == 0 && np < 16) push(5);
-  return rest == 1;
+// Column pairs per workgroup (as its binary logarithm) of the one-kernel
+// transforms, -1 where the two-pass ones are taken.  Up to 1024 rows one kernel
+// is the faster at every width, with more pairs where there are workgroups to
+// spare (longer runs of memory).  us per step, two passes and one: 32x64 72 and
+// 55, 128x192 85 and 64, 225x360 122 and 112, 512x1024 210 and 196, 700x1000 244
+// and 230, 2048x512 263 and 240 (4 pairs; 244 and 262 with 2 and 1), 4096x1024
+// 755 and 720.  With 2048 rows the two are about equal up to 1024 columns, and
+// at 2048x2048 one takes 790 where two take 727.
+static int one_pass_pairs(int n, int itot) {
+  if (n > 1024) return -1;
+  return itot >= 1024 ? 2 : itot >= 256 ? 1 : 0;
 }
+
+// Powers of two have their schedules compiled in, other factors read theirs
+// (registers of the largest radix, a switch per stage: 512x1024 30 us that way,
+// 24 compiled in).
+using Any = AnySched<16, 3>;
+
+// the two passes' factors
+static bool pass_sched(int m, FftSched &sc) { return fft_sched(m, sc, Any::rmax, Any::npmax); }
 
 bool fft2_plan(int n, int itot, Fft2Plan &pl, int n1) {
   if (n < 4) return false;
   // n1 = the given factor, else the largest divisor of n not above sqrt(n)
   // that the radices cover
+  FftSched s1, s2;
   int best = -1;
   if (n1 > 0) {
-    int np1, np2;
-    unsigned long long c1, c2;
-    if (n % n1 || n1 < 2 || n / n1 < 2 || !radix_code(n1, np1, c1) ||
-        !radix_code(n / n1, np2, c2))
+    if (n % n1 || n1 < 2 || n / n1 < 2 || !pass_sched(n1, s1) || !pass_sched(n / n1, s2))
       return false;
     best = n1;
   } else {
-    for (int d = 1; d * d <= n; d++) {
-      if (n % d) continue;
-      int np1, np2;
-      unsigned long long c1, c2;
-      if (radix_code(d, np1, c1) && radix_code(n / d, np2, c2)) best = d;
-    }
+    for (int d = 2; d * d <= n; d++)
+      if (n % d == 0 && pass_sched(d, s1) && pass_sched(n / d, s2)) best = d;
   }
-  if (best < 1) return false;
+  if (best < 2) return false;
+  pl = Fft2Plan{};
   pl.n = n;
   pl.n1 = best;
   pl.n2 = n / best;
-  if (pl.n1 == 1) {  // keep both passes non-trivial only when possible
-    return false;
-  }
-  radix_code(pl.n1, pl.np1, pl.code1);
-  radix_code(pl.n2, pl.np2, pl.code2);
-  if (2 * TILE * pl.n2 > EMAXF * NTF) return false;  // pass B must fit its LDS tile
-  int G = 1;
-  for (int c = 1; c <= pl.n2; c++)
-    if (pl.n2 % c == 0 && c * TILE * pl.n1 <= EMAXF * NTF) G = c;
-  pl.G = G;
   pl.npair = (itot + 1) / 2;
-  return TILE * pl.n1 <= EMAXF * NTF;
+  if (pl.n1 > 256 || pl.n2 > 128) return false;  // the workgroups' LDS
+  int lgt = n1 > 0 ? -1 : one_pass_pairs(n, itot);
+  if (lgt >= 0 && one_pass_sched(n, pl.s1))
+    while (lgt >= 0 && (fft_threads(1 << lgt, pl.s1) > kMaxThreads ||
+                        fft_lds_bytes(1 << lgt, n) > kMaxLds))
+      lgt--;
+  else lgt = -1;
+  if (lgt >= 0) {
+    pl.one = true;
+    pl.lgt = lgt;
+    return true;
+  }
+  pass_sched(pl.n1, pl.s1);
+  pass_sched(pl.n2, pl.s2);
+  // 8 pairs, 128-byte runs: 16 measured the same (564 and 579 us for the four
+  // passes of 4096x8192, 145 both at 2048x4096), 4 slower (707 and 158)
+  pl.lgt = 3;
+  while (fft_threads(1 << pl.lgt, pl.s1) > kMaxThreads ||
+         fft_threads(2 << pl.lgt, pl.s2) > kMaxThreads)
+    pl.lgt--;
+  const int T = 1 << pl.lgt;
+  pl.G = 1;
+  for (int c = 2; c <= pl.n2; c++)
+    if (pl.n2 % c == 0 && c * T * pl.n1 <= kElems && fft_threads(c * T, pl.s1) <= kMaxThreads)
+      pl.G = c;
+  return true;
 }
-
-static dim3 grid_a(const Fft2Plan &pl) { return dim3((pl.npair + TILE - 1) / TILE, pl.n2 / pl.G); }
-static dim3 grid_b(const Fft2Plan &pl) { return dim3((pl.npair + TILE - 1) / TILE, pl.n1 / 2 + 1); }
 
 static dim3 with_z(dim3 d, int nz) { return dim3(d.x, d.y, nz); }
 
-// Compile-time length of a pass: the factor itself when it is a power of
-// two in 8..128 and the pass's sequence count is a power of two, else 0 (the
-// runtime radix schedule).
-static int p2_len(int m, int S) {
-  const bool pow2 = (m & (m - 1)) == 0 && (S & (S - 1)) == 0;
-  return pow2 && m >= 8 && m <= 128 ? m : 0;
+// f(schedule type) for the fixed schedules, else Any.
+template <class F>
+static void two_pass_sched(const FftSched &sc, F f) {
+  if (FixedSched<4, 8>::is(sc)) f(FixedSched<4, 8>{});
+  else if (FixedSched<8, 8>::is(sc)) f(FixedSched<8, 8>{});
+  else if (FixedSched<8, 16>::is(sc)) f(FixedSched<8, 16>{});
+  else f(Any{});
+}
+template <class S>
+static void poisson_forward(hipStream_t s, const Fft2Plan &pl, bool pow2, bool aligned, S src,
+                            int nz) {
+  if (pl.one) return one_pass_forward(s, pl, aligned, src, nz);
+  const int T = 1 << pl.lgt, nt = (pl.npair + T - 1) / T;
+  const dim3 ga(nt, pl.n2 / pl.G), gb(nt, pl.n1 / 2 + 1);
+  if (!aligned) SNS_FFT_LAUNCH((k_pfwd_a<Any, false, false, S>), pl.G * T, pl.s1, ga);
+  else
+    two_pass_sched(pl.s1, [&](auto sc) {
+      if (pow2) SNS_FFT_LAUNCH((k_pfwd_a<decltype(sc), true, true, S>), pl.G * T, pl.s1, ga);
+      else SNS_FFT_LAUNCH((k_pfwd_a<decltype(sc), false, true, S>), pl.G * T, pl.s1, ga);
+    });
+  two_pass_sched(pl.s2, [&](auto sc) {
+    SNS_FFT_LAUNCH((k_pfwd_b<decltype(sc), S>), 2 * T, pl.s2, gb);
+  });
 }
 
-// Launch kernel template K<L, S> with L the compile-time length of factor m
-#define SNS_P2_LAUNCH(K, L_, grid)                                                        \
-  switch (L_) {                                                                           \
-    case 8: hipLaunchKernelGGL((K<8, S>), grid, dim3(NTF), 0, s, src); break;              \
-    case 16: hipLaunchKernelGGL((K<16, S>), grid, dim3(NTF), 0, s, src); break;            \
-    case 32: hipLaunchKernelGGL((K<32, S>), grid, dim3(NTF), 0, s, src); break;            \
-    case 64: hipLaunchKernelGGL((K<64, S>), grid, dim3(NTF), 0, s, src); break;            \
-    case 128: hipLaunchKernelGGL((K<128, S>), grid, dim3(NTF), 0, s, src); break;          \
-    default: hipLaunchKernelGGL((K<0, S>), grid, dim3(NTF), 0, s, src); break;             \
-  }
+template <class S>
+static void poisson_inverse(hipStream_t s, const Fft2Plan &pl, bool aligned, S src, int nz) {
+  if (pl.one) return one_pass_inverse(s, pl, aligned, src, nz);
+  const int T = 1 << pl.lgt, nt = (pl.npair + T - 1) / T;
+  const dim3 ga(nt, pl.n2 / pl.G), gb(nt, pl.n1 / 2 + 1);
+  two_pass_sched(pl.s2, [&](auto sc) {
+    SNS_FFT_LAUNCH((k_pinv_b<decltype(sc), S>), 2 * T, pl.s2, gb);
+  });
+  if (!aligned) SNS_FFT_LAUNCH((k_pinv_a<Any, false, S>), pl.G * T, pl.s1, ga);
+  else
+    two_pass_sched(pl.s1, [&](auto sc) {
+      SNS_FFT_LAUNCH((k_pinv_a<decltype(sc), true, S>), pl.G * T, pl.s1, ga);
+    });
+}
 
 template <class S>
 static void poisson_stage(hipStream_t s, const Geo &g, const Fft2Plan &pl, bool pow2,
                           bool aligned, S src, int nz, int stage) {
-  // pass A runs G*TILE sequences of length n1, pass B up to 2*TILE of length n2
-  const int La = p2_len(pl.n1, pl.G * TILE);
-  const int Lb = p2_len(pl.n2, TILE);
-  if (stage == 0 || stage < 0) {
-    if (aligned && pow2) SNS_P2_LAUNCH(k_pfwd_a_p2, La, with_z(grid_a(pl), nz))
-    else if (aligned) SNS_P2_LAUNCH(k_pfwd_a_al, La, with_z(grid_a(pl), nz))
-    else SNS_P2_LAUNCH(k_pfwd_a, La, with_z(grid_a(pl), nz));
-    SNS_P2_LAUNCH(k_pfwd_b, Lb, with_z(grid_b(pl), nz));
-  }
+  if (stage == 0 || stage < 0) poisson_forward(s, pl, pow2, aligned, src, nz);
   if (stage == 1 || stage < 0) {
     int NT, M;
     px_shape(g.itot, NT, M);
@@ -622,11 +509,7 @@ static void poisson_stage(hipStream_t s, const Geo &g, const Fft2Plan &pl, bool 
       }
     }
   }
-  if (stage == 2 || stage < 0) {
-    SNS_P2_LAUNCH(k_pinv_b, Lb, with_z(grid_b(pl), nz));
-    if (aligned) SNS_P2_LAUNCH(k_pinv_a_al, La, with_z(grid_a(pl), nz))
-    else SNS_P2_LAUNCH(k_pinv_a, La, with_z(grid_a(pl), nz));
-  }
+  if (stage == 2 || stage < 0) poisson_inverse(s, pl, aligned, src, nz);
 }
 
 // The padded state layout: even row pitches, ux rows and the column 1 of uy

@@ -47,9 +47,9 @@ import sys
 # kernel function -> group
 GROUPS = [
     ("k_pred_rows", "pred"), ("k_pred_exp", "pred"),
-    ("k_pfwd_a", "poisson_fwd"), ("k_pfwd_b", "poisson_fwd"),
+    ("k_pfwd_a", "poisson_fwd"), ("k_pfwd_b", "poisson_fwd"), ("k_pfwd_one", "poisson_fwd"),
     ("k_poisson_x3", "poisson_x"), ("k_poisson_factor", "setup"),
-    ("k_pinv_b", "poisson_inv"), ("k_pinv_a", "poisson_inv"),
+    ("k_pinv_b", "poisson_inv"), ("k_pinv_a", "poisson_inv"), ("k_pinv_one", "poisson_inv"),
     ("k_corr", "corr"), ("k_dt_reduce", "dt_reduce"), ("k_fill_u64", "dt_reduce"),
     ("k_adv_bound", "dt_reduce"),
     ("k_dt", "dt"), ("k_lu_factor", "lu_factor"), ("k_copy", "copy"),
@@ -66,7 +66,7 @@ def short_name(full):
 
 def group_of(full):
     """Group of a kernel: its name, or a variant of it (name + "_" + suffix,
-    e.g. k_pfwd_a_p2, the power-of-two variant of k_pfwd_a)."""
+    e.g. k_yapply_rows, a variant of k_yapply)."""
     s = short_name(full)
     for k, g in GROUPS:
         if s == k or s.startswith(k + "_"):

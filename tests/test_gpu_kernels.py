@@ -147,3 +147,40 @@ def test_explicit_x_predictor_edges(sns, itot, jtot, stretch, with_t, imy):
                 assert np.array_equal(got, fields[n]), (n, np.abs(got - fields[n]).max())
             fields[n] = got
         inst.close()
+
+
+# (itot, jtot, first factor of the two passes or 0 for the rule): whole columns in
+# one kernel up to 1024 rows with 1, 2 and 4 column pairs a workgroup (compiled
+# and read schedules, one stage, odd lengths), two passes above (two and three
+# stages, factors of 16*16 and 3*9*9, a half tile of columns)
+FFT_CASES = [(4, 4, 0), (5, 6, 0), (4, 10, 0), (16, 16, 0), (31, 32, 0), (33, 75, 0), (255, 64, 0),
+             (256, 48, 0), (17, 192, 0), (257, 1000, 0), (40, 243, 0), (1023, 128, 0),
+             (1024, 320, 0), (1025, 1024, 0), (16, 1080, 0), (17, 1125, 0), (9, 2048, 0),
+             (40, 2000, 0), (5, 1458, 0), (33, 486, 243), (7, 512, 256), (18, 250, 125),
+             (6, 16384, 0)]
+
+
+@pytest.mark.parametrize("itot,jtot,n1", FFT_CASES)
+def test_transforms_by_length(sns, pinned_gauge, itot, jtot, n1):  # noqa: F811
+    """The potential to 1e-11 of the oracle's after removing its mean (the bar
+    of the other sizes), and two fused steps (padded layout) equal to the
+    reference-named functions (packed layout)."""
+    o, inst = make_pair(sns, itot, jtot, 3.0, 0, 0, seed=itot + jtot)
+    inst.set_launch(fft_n1=n1)
+    assert inst.launch()["fft_n1"] == n1 or jtot > 1024
+    o.compute_potential(1)
+    inst.compute_potential(1)
+    assert_close(interior(inst.download("psi")), interior(o.f["psi"]), 1e-11, "psi", demean=True)
+    names = ("ux", "uy", "p", "temp")
+    inst.state_alloc()
+    for n in names:
+        inst.update_boundaries(n)
+        inst.state_upload(n, inst.download(n))
+    inst.set_dt(1e-8)
+    for _ in range(2):  # T's two buffers: back in the one that holds the corners
+        inst.integrate()
+        inst.integrate_reference_order()
+    for n in names:
+        inst.update_boundaries(n)
+        assert np.array_equal(inst.state_download(n), inst.download(n)), n
+    inst.close()
