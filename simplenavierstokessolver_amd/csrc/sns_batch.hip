@@ -188,7 +188,7 @@ void lane_launch(const Lane &k, int p) {
   const int nz = (int)k.mem.size();
   const hipStream_t s = k.stream;
   const StepArgs &sh = k.shape;
-  launch_dt_batch(s, k.dt, nz);
+  if (!sh.dt_first) launch_dt_batch(s, k.dt, nz);
   if (k.impx) launch_lu_factor_batch(s, sh.lu, k.lu, nz);
   if (k.impy && sh.yf.L) launch_yfactor_batch(s, k.yf, nz);
   for (int rk = 0; rk < 3; rk++) {

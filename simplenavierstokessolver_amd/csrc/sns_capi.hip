@@ -1250,6 +1250,11 @@ void step_args(const snsg_ctx *c, const snsg_state *st, bool reduce, StepArgs &s
       if (pa.p_out) in_p = pa.p_out;
     }
   }
+  // The first kernel decides dt where that is cheap: 18 workgroups of factors
+  // read up to 2048 partials each, the predictor's, in their hundreds, 512.
+  const bool yfac = impy && sa.yf.L;
+  sa.dt_first = reduce && c->nparts <= (impx || yfac ? 2048 : 512);
+  if (sa.dt_first) (impx ? sa.lu.dt : yfac ? sa.yf.dt : sa.pred[0].dt) = sa.dt;
 }
 
 // One RK3 step with the fused kernels; dt is read from the device slot
@@ -1307,7 +1312,7 @@ extern "C" int snsg_advance(snsg_ctx *c, snsg_state *st, int nsteps) {
   step_args(c, st, true, sa);
   if ((rc = run(c, "dt_reduce", [&] { launch_adv_bound(c->stream, sa.bound); }))) return rc;
   for (int n = 0; n < nsteps; n++) {
-    if ((rc = run(c, "dt", [&] { launch_dt(c->stream, sa.dt); }))) return rc;
+    if (!sa.dt_first && (rc = run(c, "dt", [&] { launch_dt(c->stream, sa.dt); }))) return rc;
     if ((rc = integrate_fused(c, st, true))) return rc;
   }
   return 0;

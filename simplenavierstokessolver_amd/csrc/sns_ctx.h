@@ -88,6 +88,7 @@ PoisArgs pois_args(const snsg_ctx *c, const Geo &g, double gamma, const double *
 struct StepArgs {
   LuFactorArgs lu;
   DtArgs dt;
+  bool dt_first;   // the step's first kernel decides dt
   CorrArgs bound;  // advective bound of the state as it is (d_part)
   YFactorArgs yf;  // factors of the partitioned y solves (ychunk > 0)
   PredArgs pred[3];

@@ -5,6 +5,46 @@
 
 namespace sns {
 
+// Time-step decision of one instance from the partial minima of the
+// advective bound (k_corr / k_adv_bound)
+struct DtArgs {
+  const double *part;
+  int n;
+  double *dt, *time;
+  double dt_dif_x, dt_dif_y;
+  int implicitx, implicity;
+};
+
+// dt and time from the minimum m of the advective bound
+// (src/param/decide_dt.c:45-97, src/main.c:34-35).
+__device__ __forceinline__ double dt_of(const DtArgs &a, double m) {
+  const double dt_adv = m * 0.7;
+  const double dx = a.dt_dif_x, dy = a.dt_dif_y;
+  return a.implicitx ? a.implicity ? dt_adv : fmin(dt_adv, dy)
+                     : a.implicity ? fmin(dt_adv, dx) : fmin(dt_adv, fmin(dx, dy));
+}
+
+// The time step a kernel runs with: *dtp, or (dt.part set: the step's first
+// kernel) decided here, by every wave for itself from the partial minima, and
+// stored by the workgroup with `store` for the kernels that follow.  It takes
+// the place of a launch of one workgroup: us per step, with it and without,
+// 32x64 53.0 and 55.0, 225x360 110.9 and 112.6, 512x1024 192.7 and 195.5.  All
+// lanes call.
+__device__ __forceinline__ double dt_of_step(const DtArgs &a, const double *dtp, bool store) {
+  if (!a.part) return *dtp;
+  double m = a.part[0];
+#pragma unroll 8
+  for (int k = threadIdx.x & 63; k < a.n; k += 64) m = fmin(m, a.part[k]);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) m = fmin(m, __shfl_xor(m, off));
+  const double d = dt_of(a, m);
+  if (store && threadIdx.x == 0) {
+    *a.dt = d;
+    *a.time += d;
+  }
+  return d;
+}
+
 struct PredArgs {
   Geo g;
   Tables tb;
@@ -14,6 +54,7 @@ struct PredArgs {
   double *out_u, *out_v, *out_t;          // ux*, uy*, T' with boundary values
   double *q_u, *q_v, *q_t;                // x-aligned increments (set when a y solve follows)
   const double *dtp;
+  DtArgs dt;                              // dt_of_step (explicit x)
   double alpha, beta, gamma;
   int read_hist, write_hist;
   int with_temp;                          // temperature equation integrated
@@ -41,15 +82,6 @@ struct CorrArgs {
   double *red;  // per-workgroup advective-bound minima (corr_partials entries), or nullptr
 };
 
-// Time-step decision of one instance from the partial minima of the
-// advective bound (k_corr / k_adv_bound)
-struct DtArgs {
-  const double *part;
-  int n;
-  double *dt, *time;
-  double dt_dif_x, dt_dif_y;
-  int implicitx, implicity;
-};
 
 // Thomas factorisation tables of the three CN-x operators for the three
 // substages: out holds 9 groups (substage s, field f at (s*3+f)) of 3 tables
@@ -107,6 +139,7 @@ struct LuFactorArgs {
   Geo g;
   Tables tb;
   const double *dtp;
+  DtArgs dt;  // dt_of_step
   double gamma[3];
   double *out;
   int ntm;
@@ -117,6 +150,7 @@ struct LuFactorArgs {
 struct YFactorArgs {
   Geo g;
   const double *dtp;
+  DtArgs dt;  // dt_of_step
   double gamma[3];
   double *out;
   int L, S;

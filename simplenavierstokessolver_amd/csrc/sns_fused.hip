@@ -39,12 +39,11 @@ constexpr int kExpWaves = 4;
 
 template <int F, bool P2, bool FOLD, int IMY>
 __device__ __forceinline__ void pred_exp_body(const PredArgs &a, int b, int ja, int jb,
-                                              bool write_a) {
+                                              bool write_a, double dt) {
   const Geo &g = a.g;
   const int itot = g.itot;
   const int n = F == 1 ? itot - 1 : itot;
   const int i0 = F == 1 ? 2 : 1;
-  const double dt = *a.dtp;
   const LanePos p = lane_pos(1 + b * kBlockCols - 2, i0, n, itot, 0, n, 1, 63);
   const bool edge = (F == 1 && b == 0) || (b + 1) * kBlockCols >= n;
   const RowSrc<F, FOLD> q = row_src<F, FOLD>(a, ja, jb, n);
@@ -98,6 +97,7 @@ __device__ __forceinline__ void pred_exp_body(const PredArgs &a, int b, int ja, 
 template <bool P2, bool FOLD, int IMY, class S>
 __global__ void __launch_bounds__(64 * kExpWaves, 3) k_pred_exp(S src, int nfld, int ncg) {
   const PredArgs a = src.get();
+  const double dt = dt_of_step(a.dt, a.dtp, blockIdx.x == 0);
   const int w = xcd_groups(blockIdx.x, gridDim.x, kPredGroup * nfld * ncg);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int b = (w % ncg) * (blockDim.x >> 6) + wave;
@@ -106,9 +106,9 @@ __global__ void __launch_bounds__(64 * kExpWaves, 3) k_pred_exp(S src, int nfld,
   if (b * kBlockCols >= a.g.itot) return;
   const int ja = min(2 * q + 1, a.g.jtot - 1), jb = ja + 1;
   const bool write_a = ja == 2 * q + 1;
-  if (f == 0) pred_exp_body<0, P2, FOLD, IMY>(a, b, ja, jb, write_a);
-  else if (f == 1) pred_exp_body<1, P2, FOLD, IMY>(a, b, ja, jb, write_a);
-  else pred_exp_body<2, P2, FOLD, IMY>(a, b, ja, jb, write_a);
+  if (f == 0) pred_exp_body<0, P2, FOLD, IMY>(a, b, ja, jb, write_a, dt);
+  else if (f == 1) pred_exp_body<1, P2, FOLD, IMY>(a, b, ja, jb, write_a, dt);
+  else pred_exp_body<2, P2, FOLD, IMY>(a, b, ja, jb, write_a, dt);
 }
 
 // Power-of-two divisors select the variant that divides by multiplying, a psi
@@ -372,10 +372,7 @@ __global__ void __launch_bounds__(kDtThreads) k_dt(S src) {
   if (threadIdx.x != 0) return;
   for (int w = 1; w < kDtThreads / 64; w++) m = fmin(m, wm[w]);
   m = fmin(m, wm[0]);
-  const double dt_adv = m * 0.7;
-  const double dx = a.dt_dif_x, dy = a.dt_dif_y;
-  const double d = a.implicitx ? a.implicity ? dt_adv : fmin(dt_adv, dy)
-                               : a.implicity ? fmin(dt_adv, dx) : fmin(dt_adv, fmin(dx, dy));
+  const double d = dt_of(a, m);
   *a.dt = d;
   *a.time += d;
 }

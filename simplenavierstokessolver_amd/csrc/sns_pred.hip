@@ -80,7 +80,8 @@ __global__ void __launch_bounds__(NT) k_lu_factor(S src) {
   const int n = f == 1 ? g.itot - 1 : g.itot;
   // substage gamma selected without indexing (keeps the argument block in registers)
   const double gam = s == 0 ? a.gamma[0] : s == 1 ? a.gamma[1] : a.gamma[2];
-  const double pf = cn_pf(g, f, gam * (*a.dtp));
+  const double dt = dt_of_step(a.dt, a.dtp, f == 0 && s == 0);
+  const double pf = cn_pf(g, f, gam * dt);
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   // chunk product of the row matrices (rows >= 1)
   M22 T = {1., 0., 0., 1.};

@@ -116,10 +116,10 @@ __global__ void __launch_bounds__(64) k_yfactor(S src) {
   double *t = a.out + (size_t)(s * 3 + f) * a.stride;
   if (!a.onepass)
     for (int k = threadIdx.x; k < NR; k += 64) srr[k] = sal[k] = sbe[k] = sq1[k] = 0.;
+  const double dt = dt_of_step(a.dt, a.dtp, f == 0 && s == 0);
   __syncthreads();
   if (threadIdx.x == 0) {
     const double gam = s == 0 ? a.gamma[0] : s == 1 ? a.gamma[1] : a.gamma[2];
-    const double dt = *a.dtp;
     const double pf = f == 0 ? cny_pf<KIND_TEMP>(a.g, gam, dt) : cny_pf<KIND_UX>(a.g, gam, dt);
     // coefficients as src/temperature/update.c:188-197
     const double coef_ym = 1. / a.g.dy / a.g.dy, coef_yp = 1. / a.g.dy / a.g.dy;

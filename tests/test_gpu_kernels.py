@@ -184,3 +184,34 @@ def test_transforms_by_length(sns, pinned_gauge, itot, jtot, n1):  # noqa: F811
         inst.update_boundaries(n)
         assert np.array_equal(inst.state_download(n), inst.download(n)), n
     inst.close()
+
+
+# (itot, jtot, implicit x, y): partial minima at the edges of the rule (512 for
+# the explicit predictor, 2048 for the factors) and a few
+DT_CASES = [(4, 8, 0, 0), (248, 1024, 0, 0), (249, 1024, 0, 0), (248, 1024, 0, 1),
+            (16, 4096, 0, 1), (16, 4320, 0, 1), (16, 4096, 1, 0), (16, 4320, 1, 0),
+            (300, 24, 1, 1)]
+
+
+@pytest.mark.parametrize("itot,jtot,imx,imy", DT_CASES)
+def test_time_step_decided_by_first_kernel(sns, itot, jtot, imx, imy):
+    """Three steps of the time loop, whose first kernels decide dt, against
+    dt decided on the host before each step: dt, time and fields equal."""
+    def make():
+        inst = sns.Instance(itot, jtot, stretch=3.0, Ra=1e6, Pr=2.0, implicitx=imx, implicity=imy)
+        inst.state_alloc()
+        inst.state_init_temperature(itot + jtot, 1e-2)
+        return inst
+    a, b = make(), make()
+    a.advance(3)
+    t = 0.0
+    for _ in range(3):
+        dt = sns.decide_dt(b.g, 1e6, 2.0, b.state_dt_adv_raw(), imx, imy)
+        b.set_dt(dt)
+        b.integrate()
+        t += dt
+    assert a.get_time() == (t, dt)
+    for n in ("ux", "uy", "p", "temp"):
+        assert np.array_equal(a.state_download(n), b.state_download(n)), n
+    a.close()
+    b.close()
