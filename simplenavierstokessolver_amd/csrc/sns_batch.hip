@@ -420,14 +420,20 @@ struct Pooled {
 };
 
 // A lane of the engine: its jobs (in the order of the lane's members), the
-// step in flight, and the set-up events of jobs that joined since the last
-// step.
+// steps in flight, and the set-up events of jobs that joined since the last
+// step.  A second step is enqueued behind the running one, so the device does
+// not wait for the engine between them (four jobs of 128x256 to 512x1024, 100 to
+// 150 steps: 113 ms with their downloads, 118 with one step at a time), unless the
+// membership changes there: a job joined, or one of the running step's ends.
+constexpr int kAhead = 2;
 struct ServeLane {
   Lane k;
   std::vector<Job *> jobs;
-  bool busy = false, dirty = false;
+  bool dirty = false;
+  int inflight = 0, head = 0;  // steps enqueued; slot of the oldest
+  size_t nmem[kAhead] = {};    // its members, the first of jobs
   int parity = 0;
-  hipEvent_t t0 = nullptr, t1 = nullptr;
+  hipEvent_t t0[kAhead] = {}, t1[kAhead] = {};
   std::vector<hipEvent_t> waits;
 };
 
@@ -551,8 +557,10 @@ static int engine_admit(snsg_server *s, bool &progressed) {
     if (!L) {
       L = new ServeLane();
       if ((rc = lane_init(L->k, j->c))) return rc;
-      HIPCHECK(hipEventCreate(&L->t0));
-      HIPCHECK(hipEventCreate(&L->t1));
+      for (int n = 0; n < kAhead; n++) {
+        HIPCHECK(hipEventCreate(&L->t0[n]));
+        HIPCHECK(hipEventCreate(&L->t1[n]));
+      }
     }
     L->k.mem.push_back({j->c, &j->st});
     L->jobs.push_back(j);
@@ -571,18 +579,20 @@ static int engine_admit(snsg_server *s, bool &progressed) {
   }
 }
 
-// Collects the lanes whose step has finished; jobs that reached their step
+// Collects the lanes whose oldest step has finished; jobs that reached their step
 // count leave their lane (kept for download, or pooled for reuse).
 static int engine_collect(snsg_server *s, bool &progressed) {
   for (auto &kv : s->lanes) {
     ServeLane &L = *kv.second;
-    if (!L.busy) continue;
-    const hipError_t q = hipEventQuery(L.t1);
+    if (!L.inflight) continue;
+    const hipError_t q = hipEventQuery(L.t1[L.head]);
     if (q == hipErrorNotReady) continue;
     if (q != hipSuccess) return set_err((int)q, "server: lane step");
     float ms = 0.f;
-    HIPCHECK(hipEventElapsedTime(&ms, L.t0, L.t1));
-    L.busy = false;
+    HIPCHECK(hipEventElapsedTime(&ms, L.t0[L.head], L.t1[L.head]));
+    const size_t nmem = L.nmem[L.head];
+    L.head = (L.head + 1) % kAhead;
+    L.inflight--;
     progressed = true;
     std::vector<Job *> left;
     std::vector<Member> mem;
@@ -592,6 +602,11 @@ static int engine_collect(snsg_server *s, bool &progressed) {
       const Clock::time_point now = Clock::now();
       for (size_t m = 0; m < L.jobs.size(); m++) {
         Job *j = L.jobs[m];
+        if (m >= nmem) {  // joined while the step ran
+          left.push_back(j);
+          mem.push_back(L.k.mem[m]);
+          continue;
+        }
         j->done++;
         s->steps++;
         s->cell_steps += (double)j->cfg.itot * (double)j->cfg.jtot;
@@ -634,25 +649,32 @@ static int engine_collect(snsg_server *s, bool &progressed) {
   return 0;
 }
 
-// Starts the next step of every idle lane that has jobs.
+// Enqueues steps of every lane that has jobs, up to kAhead.
 static int engine_launch(snsg_server *s, bool &progressed) {
   for (auto &kv : s->lanes) {
     ServeLane &L = *kv.second;
-    if (L.busy || L.jobs.empty()) continue;
+    if (L.jobs.empty()) continue;
     int rc;
-    if (L.dirty) {
+    if (L.dirty && L.inflight == 0) {
       if ((rc = lane_build(L.k))) return rc;
       L.parity = 0;
       L.dirty = false;
     }
-    for (hipEvent_t e : L.waits) HIPCHECK(hipStreamWaitEvent(L.k.stream, e, 0));
-    L.waits.clear();
-    HIPCHECK(hipEventRecord(L.t0, L.k.stream));
-    if ((rc = lane_step(L.k, L.parity, true))) return rc;
-    HIPCHECK(hipEventRecord(L.t1, L.k.stream));
-    if (L.k.with_temp) L.parity ^= 1;
-    L.busy = true;
-    progressed = true;
+    while (!L.dirty && L.inflight < kAhead) {
+      bool ends = false;
+      for (const Job *j : L.jobs) ends = ends || j->done + L.inflight >= j->nsteps;
+      if (ends) break;
+      for (hipEvent_t e : L.waits) HIPCHECK(hipStreamWaitEvent(L.k.stream, e, 0));
+      L.waits.clear();
+      const int slot = (L.head + L.inflight) % kAhead;
+      HIPCHECK(hipEventRecord(L.t0[slot], L.k.stream));
+      if ((rc = lane_step(L.k, L.parity, true))) return rc;
+      HIPCHECK(hipEventRecord(L.t1[slot], L.k.stream));
+      L.nmem[slot] = L.jobs.size();
+      if (L.k.with_temp) L.parity ^= 1;
+      L.inflight++;
+      progressed = true;
+    }
   }
   return 0;
 }
@@ -678,7 +700,7 @@ static void engine_main(snsg_server *s) {
     }
     if (stopping) {
       bool busy = false;
-      for (auto &kv : s->lanes) busy = busy || kv.second->busy;
+      for (auto &kv : s->lanes) busy = busy || kv.second->inflight;
       if (!busy || rc) return;
     }
     if (!progressed) std::this_thread::sleep_for(std::chrono::microseconds(20));
@@ -864,8 +886,10 @@ extern "C" int snsg_server_destroy(snsg_server *s) {
   (void)hipSetDevice(s->device);
   for (auto &kv : s->lanes) {
     lane_free(kv.second->k);
-    if (kv.second->t0) (void)hipEventDestroy(kv.second->t0);
-    if (kv.second->t1) (void)hipEventDestroy(kv.second->t1);
+    for (int n = 0; n < kAhead; n++) {
+      if (kv.second->t0[n]) (void)hipEventDestroy(kv.second->t0[n]);
+      if (kv.second->t1[n]) (void)hipEventDestroy(kv.second->t1[n]);
+    }
     delete kv.second;
   }
   for (auto &kv : s->pool) destroy_instance(kv.second.c, &kv.second.st);

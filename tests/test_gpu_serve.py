@@ -143,3 +143,27 @@ def test_server_slots_bound_the_active_jobs(sns):
     assert st["completed"] == len(SPECS) and st["active_peak"] == 2
     assert st["steps"] == sum(s[2] for s in SPECS)
     srv.close()
+
+
+def test_server_job_joins_running_lane(sns):
+    """A job submitted while a step of its class is in flight takes its own
+    steps only: it and the running job end bitwise where each ends alone."""
+    specs = [(64, 128, 600, 1e7, 1.0, 1, 0, 3), (64, 128, 25, 1e8, 0.7, 1, 0, 4),
+             (64, 128, 26, 1e6, 2.0, 1, 0, 5)]
+    srv = sns.Server(10 ** 9)
+    ids = [submit(srv, specs[0], keep=True)]
+    deadline = time.time() + 60
+    while srv.status(ids[0])[1] < 5 and time.time() < deadline:
+        time.sleep(0.001)
+    for spec in specs[1:]:
+        ids.append(submit(srv, spec, keep=True))
+        time.sleep(0.003)
+    for jid, spec in zip(ids, specs):
+        srv.wait(jid, 120.0)
+        assert srv.status(jid) == (2, spec[2])
+        ref = alone(sns, spec)
+        for n in FIELDS:
+            assert same(srv.download(jid, n), ref[n]), (spec, n)
+        assert srv.job_time(jid) == ref["time"]
+        srv.release(jid)
+    srv.close()
