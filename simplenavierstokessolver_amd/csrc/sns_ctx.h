@@ -2,6 +2,7 @@
 // C-ABI translation units share (internal).
 #pragma once
 #include <stddef.h>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -51,6 +52,9 @@ struct snsg_ctx {
   double *d_lu = nullptr;
   int lu_ntm = 0;
   double *d_time = nullptr;
+  // packed rows of a field on their way to or from the host (pack_doubles)
+  double *d_pack = nullptr;
+  std::mutex pack_mu;
   size_t mem = 0;  // device bytes held by the context and its state
   double dt_dif_x = 0., dt_dif_y = 0.;
   // timing

@@ -379,6 +379,21 @@ void launch_fill_u64(hipStream_t s, unsigned long long *p, unsigned long long v,
   hipLaunchKernelGGL(k_fill_u64, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, p, v, n);
 }
 
+// Rows of `width` values from one pitch to another.
+__global__ void __launch_bounds__(kBlock) k_copy_rows(const double *__restrict__ src, size_t sp,
+                                                      double *__restrict__ dst, size_t dp,
+                                                      size_t width) {
+  const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x, j = blockIdx.y;
+  if (i < width) dst[j * dp + i] = src[j * sp + i];
+}
+
+// rows <= 65535
+void launch_copy_rows(hipStream_t s, const double *src, size_t sp, double *dst, size_t dp,
+                      size_t width, size_t rows) {
+  hipLaunchKernelGGL(k_copy_rows, dim3((unsigned)((width + kBlock - 1) / kBlock), (unsigned)rows),
+                     dim3(kBlock), 0, s, src, sp, dst, dp, width);
+}
+
 // Plain device copy of n 16-byte words (grid-stride, one load and one store
 // per word).
 __global__ void __launch_bounds__(kBlock) k_copy(const double2 *__restrict__ src,

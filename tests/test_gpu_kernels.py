@@ -215,3 +215,18 @@ def test_time_step_decided_by_first_kernel(sns, itot, jtot, imx, imy):
         assert np.array_equal(a.state_download(n), b.state_download(n)), n
     a.close()
     b.close()
+
+
+# one field in one piece, and in several with a ragged last one (8 MiB pieces)
+@pytest.mark.parametrize("itot,jtot", [(4, 4), (33, 75), (700, 1620), (8192, 270)])
+def test_state_fields_to_and_from_the_host(sns, itot, jtot):
+    """Every value of an uploaded field comes back, and the padding of the
+    device rows is not part of it."""
+    inst = sns.Instance(itot, jtot)
+    inst.state_alloc()
+    rng = np.random.default_rng(itot)
+    for n in ("ux", "uy", "p", "temp"):
+        a = rng.standard_normal(inst.shape(n))
+        inst.state_upload(n, a)
+        assert np.array_equal(inst.state_download(n), a), n
+    inst.close()
