@@ -7,8 +7,9 @@
 // Crank-Nicolson system in x of both rows (src/temperature/update.c:124-156,
 // src/fluid/update_velocity.c:231-270, 381-414) with the shared LU tables.
 //
-// What bounds it on large grids is neither the HBM bytes (88 B per cell; 4.0
-// TB/s at 4096x8192) nor the arithmetic, but the way from the L2: the three
+// What bounds it on large grids is neither the HBM bytes (88 B per cell, 98.7
+// folded; with what is read twice 4.6 GB and 4.5 TB/s on average at 4096x8192)
+// nor the arithmetic, but the way from the L2: the three
 // fields' workgroups read 18 rows for each row, and a run of columns that
 // does not start on a cache line costs a line more.  Evaluating one block of
 // a wave's own contiguous columns after the other, so that the lines at the
@@ -267,9 +268,9 @@ __device__ __forceinline__ void pred_stencils(const PredArgs &a, const RowSrc<F,
 }
 
 // The substage-start values of the own field in rows ja, jb (corrected as in
-// raw_fold when folded), read again: the rows are in the caches since the
-// stencil phase, and the registers that would hold them (40 a thread) are
-// worth more there.
+// raw_fold when folded), read again: the registers that would hold them (40 a
+// thread, and blocks unrolled to index them) cost more.  On wide grids the rows
+// are out of the L2 by then (0.8 GB per launch at 4096x8192).
 template <int F, bool P2, bool FOLD>
 __device__ __forceinline__ void own_load(const PredArgs &a, const RowSrc<F, FOLD> &q,
                                          const LanePos &p, double dt, double2 &oa, double2 &ob) {
