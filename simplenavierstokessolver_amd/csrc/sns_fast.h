@@ -190,9 +190,6 @@ struct TempPt {
 struct CellX {
   double dxc, rdxc, dxc_p, rdxc_p, dxf, rdxf, c_xm, c_xp;
 };
-// LANE: the lanes hold consecutive columns, so the gradient at the left face
-// of column i is the one the lane of column i-1 forms at its right face,
-// bit for bit (same operands, same operations); it is taken from there.
 // The x-gradients at the faces of cell i, dtdx_xm = (T(i)-T(i-1))/DXC(i) and
 // dtdx_xp = (T(i+1)-T(i))/DXC(i+1), are given (the t_xm, t_xp entries of v
 // are not read): a kernel holding consecutive columns forms each face
