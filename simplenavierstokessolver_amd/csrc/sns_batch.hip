@@ -109,13 +109,18 @@ int lane_build(Lane &k) {
     host.resize(off + bytes);
     return off;
   };
+  // one launch serves all members: it may divide by multiplying only where
+  // every one of them has powers of two for divisors (the division sequence
+  // gives those members the same bits)
+  bool p2 = true;
+  for (const Member &m : k.mem) p2 = p2 && pow2_division(m.c->tab);
   std::vector<StepArgs> sa[2];
   for (int p = 0; p < 2; p++) {
     sa[p].resize(nz);
     for (size_t m = 0; m < nz; m++) {
       snsg_state s = *k.mem[m].st;
       if (p == 1 && k.with_temp) std::swap(s.temp, s.temp_alt);
-      step_args(k.mem[m].c, &s, true, sa[p][m]);
+      step_args(k.mem[m].c, &s, true, p2, sa[p][m]);
     }
   }
   for (size_t m = 0; m < nz; m++) k.temp0[m] = k.mem[m].st->temp;
@@ -507,7 +512,7 @@ static int engine_setup(snsg_server *s, Job *j, bool reuse) {
       (rc = snsg_state_init_temperature(j->c, &j->st, j->seed, j->amplitude)))
     return rc;
   StepArgs sa;
-  step_args(j->c, &j->st, true, sa);
+  step_args(j->c, &j->st, true, pow2_division(j->c->tab), sa);
   launch_adv_bound(j->c->stream, sa.bound);
   if ((rc = check_launch("server: advective bound"))) return rc;
   if (!j->ready) HIPCHECK(hipEventCreateWithFlags(&j->ready, hipEventDisableTiming));

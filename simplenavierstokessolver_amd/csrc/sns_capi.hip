@@ -592,6 +592,7 @@ PoisArgs pois_args(const snsg_ctx *c, const Geo &g, double gamma, const double *
   PoisArgs a;
   a.g = g;
   a.tb = c->tab;
+  a.tb.pow2 = pow2_division(c->tab);
   a.pl = c->plan;
   a.gamma = gamma;
   a.dtp = c->d_dt;
@@ -1196,7 +1197,7 @@ int step_prepare(snsg_ctx *c) {
   return 0;
 }
 
-void step_args(const snsg_ctx *c, const snsg_state *st, bool reduce, StepArgs &sa) {
+void step_args(const snsg_ctx *c, const snsg_state *st, bool reduce, bool p2, StepArgs &sa) {
   const Geo &g = c->geo_st;
   const bool impx = c->treat.implicitx, impy = c->treat.implicity;
   const bool with_temp = c->cfg.with_temperature != 0;
@@ -1238,6 +1239,7 @@ void step_args(const snsg_ctx *c, const snsg_state *st, bool reduce, StepArgs &s
     PredArgs &pa = sa.pred[rk];
     pa.g = g;
     pa.tb = c->tab;
+    pa.tb.pow2 = p2;
     pa.tr = c->treat;
     pa.ux = in_u; pa.uy = in_v; pa.p = in_p; pa.temp = temp;
     pa.hist_ux = st->srcuxa; pa.hist_uy = st->srcuya; pa.hist_t = st->srctempa;
@@ -1261,6 +1263,7 @@ void step_args(const snsg_ctx *c, const snsg_state *st, bool reduce, StepArgs &s
     double *outs[3] = {temp_alt, out_u, out_v};
     for (int f = 0; f < 3; f++) sa.y[rk][f] = y_args(c, g, rk, f, ins[f], c->d_qf[f], outs[f]);
     sa.pois[rk] = pois_args(c, g, c->cfg.gamma[rk], out_u, out_v, st->psi);
+    sa.pois[rk].tb.pow2 = p2;
     sa.corr_on[rk] = !fold || rk == 2;
     CorrArgs &ca = sa.corr[rk];
     ca.g = g;
@@ -1292,7 +1295,7 @@ static int integrate_fused(snsg_ctx *c, snsg_state *st, bool reduce) {
   if (c->geo_st.jtot < 2) return set_err(SNSG_E_SIZE, "fused step: jtot must be at least 2");
   if ((rc = step_prepare(c))) return rc;
   StepArgs sa;
-  step_args(c, st, reduce, sa);
+  step_args(c, st, reduce, pow2_division(c->tab), sa);
   const bool impx = c->treat.implicitx, impy = c->treat.implicity;
   const bool with_temp = c->cfg.with_temperature != 0;
   if (impx && (rc = run(c, "lu_factor", [&] { launch_lu_factor(c->stream, sa.lu); }))) return rc;
@@ -1337,7 +1340,7 @@ extern "C" int snsg_advance(snsg_ctx *c, snsg_state *st, int nsteps) {
   int rc;
   if ((rc = step_prepare(c))) return rc;
   StepArgs sa;
-  step_args(c, st, true, sa);
+  step_args(c, st, true, pow2_division(c->tab), sa);
   if ((rc = run(c, "dt_reduce", [&] { launch_adv_bound(c->stream, sa.bound); }))) return rc;
   for (int n = 0; n < nsteps; n++) {
     if (!sa.dt_first && (rc = run(c, "dt", [&] { launch_dt(c->stream, sa.dt); }))) return rc;

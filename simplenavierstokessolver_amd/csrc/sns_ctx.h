@@ -89,6 +89,8 @@ PoisArgs pois_args(const snsg_ctx *c, const Geo &g, double gamma, const double *
 // state st, with st->temp and st->temp_alt as they are at the start of the
 // step (T and T' trade places after every substage).  `reduce`: the last
 // correction stores the advective-bound minima for the next step in d_part.
+// `p2`: the kernels divide by multiplying (Tables::pow2 of the blocks; every
+// instance of a launch must allow it).
 struct StepArgs {
   LuFactorArgs lu;
   DtArgs dt;
@@ -123,4 +125,4 @@ struct LaunchKey {
 };
 LaunchKey launch_key(int itot, int jtot, const snsg_launch &req);
 LaunchKey launch_key(const snsg_ctx *c);
-void step_args(const snsg_ctx *c, const snsg_state *st, bool reduce, StepArgs &sa);
+void step_args(const snsg_ctx *c, const snsg_state *st, bool reduce, bool p2, StepArgs &sa);

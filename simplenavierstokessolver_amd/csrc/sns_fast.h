@@ -89,7 +89,8 @@ struct Tables {
   double u_dxc, u_rdxc, u_dxf, u_rdxf, u_cT, u_cU;
   // Set when every divisor of the stencils (DXF, DXC of all columns and dy)
   // is a power of two: the kernels then divide by multiplying with the
-  // tabulated reciprocal (see dv).
+  // tabulated reciprocal (see dv).  In a launch's arguments: whether it does
+  // so, which is the choice of all its instances (step_args).
   int pow2;
   // Set when the Poisson row coefficients the x substitutions use are each
   // one value bit for bit: pl(I) for rows 1..itot-1 (plc) and pu(I) for rows
@@ -124,8 +125,9 @@ struct Tables {
 };
 
 // Host: whether the kernels take the power-of-two division path for these
-// tables (SNSG_EXACT_DIV=1 keeps the division sequence; read at every
-// launch, both paths return the same bits).
+// tables (SNSG_EXACT_DIV=1 keeps the division sequence; read at every call,
+// and when a batch's or lane's argument tables are built; both paths return
+// the same bits).
 inline bool pow2_division(const Tables &tb) {
   const char *ex = getenv("SNSG_EXACT_DIV");
   return tb.pow2 && !(ex && strcmp(ex, "1") == 0);

@@ -120,7 +120,7 @@ static void pred_exp_launch(hipStream_t s, const PredArgs &shape, S src, int nz)
   const int ncg = (nb + kExpWaves - 1) / kExpWaves, waves = (nb + ncg - 1) / ncg;
   const int nfld = shape.with_temp ? 3 : 2;
   const dim3 grid((g.jtot + 1) / 2 * nfld * ncg, 1, nz), block(64 * waves);
-  const bool p2 = pow2_division(shape.tb), fold = shape.psi != nullptr;
+  const bool p2 = shape.tb.pow2, fold = shape.psi != nullptr;
   const bool imy = shape.tr.implicity;  // excludes fold
 #define SNS_CALL(P2, FOLD, IMY) \
   hipLaunchKernelGGL((k_pred_exp<P2, FOLD, IMY, S>), grid, block, 0, s, src, nfld, ncg)

@@ -521,13 +521,12 @@ static bool pair_layout(const PoisArgs &a) {
 }
 
 void launch_poisson(hipStream_t s, const PoisArgs &a, int stage) {
-  poisson_stage(s, a.g, a.pl, pow2_division(a.tb), pair_layout(a), ArgOne<PoisArgs>{a}, 1,
-                stage);
+  poisson_stage(s, a.g, a.pl, a.tb.pow2, pair_layout(a), ArgOne<PoisArgs>{a}, 1, stage);
 }
 
 void launch_poisson_batch(hipStream_t s, const PoisArgs &shape, const PoisArgs *dev, int nz,
                           int stage) {
-  poisson_stage(s, shape.g, shape.pl, pow2_division(shape.tb), pair_layout(shape),
+  poisson_stage(s, shape.g, shape.pl, shape.tb.pow2, pair_layout(shape),
                 arg_batch<PoisArgs>(dev), nz, stage);
 }
 

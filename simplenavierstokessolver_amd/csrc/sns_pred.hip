@@ -492,7 +492,7 @@ static void pred_rows_select(hipStream_t s, const PredArgs &shape, S src, int nz
 // psi argument the one that applies the previous substage's correction.
 template <class S>
 static void pred_rows_dispatch(hipStream_t s, const PredArgs &shape, S src, int nz) {
-  const bool p2 = pow2_division(shape.tb), fold = shape.psi != nullptr;
+  const bool p2 = shape.tb.pow2, fold = shape.psi != nullptr;
   const bool imy = shape.tr.implicity;  // excludes fold
   if (p2 && fold) pred_rows_select<true, true, 0>(s, shape, src, nz);
   else if (p2 && imy) pred_rows_select<true, false, 1>(s, shape, src, nz);

@@ -95,3 +95,31 @@ def test_batch_member_advanced_alone(sns):
     batch.close()
     for i in insts + refs:
         i.close()
+
+
+# members of one class whose first has powers of two for every divisor and
+# whose second has not, and one with the same sizes again (the kernels of a
+# class are launched once for all members)
+@pytest.mark.parametrize("itot,jtot,imx,imy", [(64, 128, 1, 0), (64, 128, 0, 0), (64, 128, 1, 1),
+                                               (64, 128, 0, 1), (32, 2048, 1, 0)])
+def test_batch_mixes_uniform_and_stretched(sns, itot, jtot, imx, imy):
+    """The members' divisors decide together how a class divides: a uniform
+    member listed first leaves a stretched one bitwise where it ends alone."""
+    ms = [(itot, jtot, stretch, 1e8, 1.3, imx, imy, True, seed)
+          for stretch, seed in ((float(itot), 1), (3.0, 2), (float(itot), 3))]
+    insts = [make(sns, m) for m in ms]
+    refs = [make(sns, m) for m in ms]
+    for i, pow2 in zip(insts, (True, False, True)):
+        spacings = list(i.g["dxf"]) + list(i.g["dxc"]) + [2.0 / jtot]
+        assert all(np.frexp(v)[0] == 0.5 for v in spacings) == pow2
+    batch = sns.Batch(insts)
+    assert batch.classes() == 1
+    batch.advance(4)
+    for r in refs:
+        r.advance(4)
+    batch.sync()
+    for inst, ref, m in zip(insts, refs, ms):
+        check(inst, ref, m)
+    batch.close()
+    for i in insts + refs:
+        i.close()

@@ -167,3 +167,27 @@ def test_server_job_joins_running_lane(sns):
         assert srv.job_time(jid) == ref["time"]
         srv.release(jid)
     srv.close()
+
+
+def test_server_mixes_uniform_and_stretched(sns):
+    """Jobs of one class on a uniform grid (powers of two for every divisor)
+    and a stretched one: the stretched job, which outlasts the uniform one
+    that was first in the lane, ends bitwise where it ends alone."""
+    specs = [(64, 128, 40, 1e8, 1.0, 1, 0, 3), (64, 128, 60, 1e7, 1.5, 1, 0, 4)]
+    srv = sns.Server(10 ** 9)
+    ids = [srv.submit(s[0], s[1], s[2], Ra=s[3], Pr=s[4], implicitx=s[5], implicity=s[6],
+                      seed=s[7], amplitude=1e-3, stretch=stretch, keep=True)
+           for s, stretch in zip(specs, (64.0, 3.0))]
+    for jid, spec, stretch in zip(ids, specs, (64.0, 3.0)):
+        srv.wait(jid, 120.0)
+        inst = sns.Instance(spec[0], spec[1], stretch=stretch, Ra=spec[3], Pr=spec[4],
+                            implicitx=1, implicity=0)
+        inst.state_alloc()
+        inst.state_init_temperature(spec[7], 1e-3)
+        inst.advance(spec[2])
+        for n in FIELDS:
+            assert same(srv.download(jid, n), inst.state_download(n)), (spec, n)
+        assert srv.job_time(jid) == inst.get_time()
+        inst.close()
+        srv.release(jid)
+    srv.close()
