@@ -301,6 +301,11 @@ static double *scratch_addr(int device) {
   return it == g_scratch_addr.end() ? nullptr : it->second;
 }
 
+// Packed rows of copy_field: a field, 8 MiB at most (128 rows of 8192 columns)
+static size_t pack_doubles(int itot, int jtot) {
+  return std::min((size_t)(itot + 2) * (jtot + 2), (size_t)1 << 20);
+}
+
 extern "C" int snsg_create(int device, const snsg_config *cfg, const double *dxf,
                            const double *dxc, snsg_ctx **out) {
   if (!cfg || !dxf || !dxc || !out) return set_err(SNSG_E_ARG, "snsg_create: null argument");
@@ -339,6 +344,7 @@ extern "C" int snsg_create(int device, const snsg_config *cfg, const double *dxf
       {(void **)&c->d_q, sizeof(double) * (size_t)(itot + 1) * jtot},
       {(void **)&c->d_qy, sizeof(double) * (size_t)(itot + 1) * jtot},
       {(void **)&c->d_red, sizeof(unsigned long long)},
+      {(void **)&c->d_pack, sizeof(double) * pack_doubles(itot, jtot)},
       {(void **)&c->d_tab, sizeof(double) * kTables * stride},
       {(void **)&c->d_tab2, sizeof(double2) * kTables2 * stride},
       {(void **)&c->d_pfac, sizeof(double) * nfac},
@@ -805,11 +811,6 @@ static int alloc_c(snsg_ctx *c, double **p) {
   return rc;
 }
 
-// Packed rows of copy_field: a field, 8 MiB at most (128 rows of 8192 columns)
-static size_t pack_doubles(int itot, int jtot) {
-  return std::min((size_t)(itot + 2) * (jtot + 2), (size_t)1 << 20);
-}
-
 extern "C" int snsg_state_alloc(snsg_ctx *c, snsg_state *st) {
   if (!c || !st) return set_err(SNSG_E_ARG, __func__);
   HIPCHECK(hipSetDevice(c->device));
@@ -818,9 +819,6 @@ extern "C" int snsg_state_alloc(snsg_ctx *c, snsg_state *st) {
   st->ld_ux = c->geo_st.pu;
   st->ld_c = c->geo_st.pc;
   int rc;
-  if (!c->d_pack && (rc = ctx_alloc((void **)&c->d_pack, sizeof(double) * pack_doubles(itot, jtot),
-                                    &c->mem)))
-    return rc;
   if ((rc = ctx_alloc((void **)&st->ux, bytes_ux(c), &c->mem))) return rc;
   if ((rc = alloc_c(c, &st->uy))) return rc;
   if ((rc = alloc_c(c, &st->p))) return rc;
@@ -910,11 +908,12 @@ extern "C" int snsg_instance_bytes(const snsg_config *cfg, size_t *bytes) {
   n += d * itot + d * (itot + 1) + d + d + d * (jtot / 2 + 1) + z * jtot;
   n += z * itot * (jtot / 2 + 1) + z * fft2_work(pl);
   n += 2 * d * (itot + 1) * jtot + sizeof(unsigned long long);
+  n += d * pack_doubles((int)itot, (int)jtot);
   n += d * kTables * stride + z * kTables2 * stride;
   n += d * poisson_factor_doubles((int)itot, (int)jtot) + d * 2 * (size_t)poisson_factor_entries((int)itot);
   // snsg_state_alloc
   n += 2 * d * pu * (jtot + 2) + 7 * d * (pc * (jtot + 2) + 16);
-  n += d * (itot - 1) * jtot + 2 * d * itot * jtot + d * pack_doubles((int)itot, (int)jtot);
+  n += d * (itot - 1) * jtot + 2 * d * itot * jtot;
   // first fused step
   if (cfg->implicity) {
     n += d * (2 * itot + itot - 1) * jtot;
@@ -957,6 +956,8 @@ static int state_field(const snsg_ctx *c, const snsg_state *st, int field, doubl
 // A field between the padded device rows and the caller's packed ones, through
 // packed rows on the device: a copy of pitched rows from or to pageable memory
 // goes row by row (26 MB of fields, 128x256 to 512x1024, in 70 ms; 5 ms so).
+// The rows belong to the instance, not to a state: any state of its grid may
+// be given.
 static int copy_field(snsg_ctx *c, double *dev, size_t pitch, size_t width, size_t rows,
                       double *host, bool up) {
   HIPCHECK(hipSetDevice(c->device));

@@ -230,3 +230,24 @@ def test_state_fields_to_and_from_the_host(sns, itot, jtot):
         inst.state_upload(n, a)
         assert np.array_equal(inst.state_download(n), a), n
     inst.close()
+
+
+def test_state_copies_need_no_state_of_the_instance(sns):
+    """The rows that state copies go through are the instance's from the start:
+    an instance without a state of its own copies the state of another one of
+    its grid, and freeing a state gives back what allocating it took."""
+    a, b = sns.Instance(40, 60), sns.Instance(40, 60)
+    before = a.memory(), b.memory()
+    a.state_alloc()
+    taken = a.memory() - before[0]
+    b.state_alloc()
+    assert b.L.snsg_state_free(b.ctx, b.state) == 0
+    assert taken > 0 and b.memory() == before[1]
+    b.state = a.state
+    f = np.random.default_rng(1).standard_normal(a.shape("ux"))
+    b.state_upload("ux", f)
+    assert np.array_equal(b.state_download("ux"), f)
+    assert np.array_equal(a.state_download("ux"), f)
+    b.state = None
+    a.close()
+    b.close()
