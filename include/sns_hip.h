@@ -235,7 +235,9 @@ typedef struct {
                            0 (the rule): with explicit y the predictors of
                            substages 2 and 3 apply the previous substage's
                            correction to the fields as they load them (the
-                           same operations, so the same bits) */
+                           same operations, so the same bits), except with
+                           implicit x above 2048 columns whose spacings are
+                           not powers of two */
 } snsg_launch;
 /* SNSG_E_ARG for a value outside the ranges above, SNSG_E_SIZE for one the
  * grid does not admit (a factor that does not divide jtot or whose FFT pass

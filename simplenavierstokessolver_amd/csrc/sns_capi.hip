@@ -1226,13 +1226,14 @@ void step_args(const snsg_ctx *c, const snsg_state *st, bool reduce, bool p2, St
   sa.bound.red = c->d_part;
   sa.yf = yfactor_args(c, g);
   double *temp = st->temp, *temp_alt = st->temp_alt;
-  // Folded corrections (explicit y): substage 1 predicts from
+  // Folded corrections (explicit y, pred_folds): substage 1 predicts from
   // (ux, uy, p) into (ux*, uy*) and stops at psi; substage 2's predictor
   // corrects ux*, uy* and p with that psi as it loads them, predicts into
   // (ux, uy) and stores the corrected p in p_alt; substage 3 does the same
   // from (ux, uy, p_alt) into (ux*, uy*) and p, and its correction kernel
   // writes ux, uy, p as in the split sequence.
-  const bool fold = !impy && !c->launch.split_corr;
+  const bool fold =
+      !impy && !c->launch.split_corr && (!impx || pred_folds(g.itot, g.jtot, p2));
   double *in_u = st->ux, *in_v = st->uy, *out_u = st->ux_star, *out_v = st->uy_star;
   double *in_p = st->p;
   for (int rk = 0; rk < 3; rk++) {

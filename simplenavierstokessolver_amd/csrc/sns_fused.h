@@ -176,6 +176,9 @@ void launch_ypart_fields_batch(hipStream_t s, const YArgs &shape, const YArgs *d
                                int nf);
 
 bool pred_impx_supported(int itot);
+// whether the implicit-x predictor may apply the previous substage's
+// correction (p2: it divides by multiplying)
+bool pred_folds(int itot, int jtot, bool p2);
 int lu_table_entries(int itot, int jtot);
 void launch_lu_factor(hipStream_t s, const LuFactorArgs &a);
 // predictor of one substage; a.lu, a.ntm: the LU tables when implicitx

@@ -407,7 +407,7 @@ __device__ __forceinline__ void pred_rows_body(const PredArgs &a, PredRowsLds<NT
 // FOLD: the fields are corrected as they are loaded (raw_fold).  IMY: a y
 // solve follows, the increments are the output.
 template <int NT, int M, bool P2, bool FOLD, int IMY, class S>
-__global__ void __launch_bounds__(NT, (pred_waves<P2, FOLD, NT>())) k_pred_rows(S src, int nfld) {
+__global__ void __launch_bounds__(NT, (pred_waves<P2, FOLD>())) k_pred_rows(S src, int nfld) {
   const PredArgs a = src.get();
   extern __shared__ double lds_raw[];
   PredRowsLds<NT, M> &L = *reinterpret_cast<PredRowsLds<NT, M> *>(lds_raw);
@@ -460,6 +460,16 @@ RowShape row_shape(int itot, int jtot) {
 
 bool pred_impx_supported(int itot) { return row_shape(itot, 4).NT > 0; }
 
+// With the division sequence the folded kernel needs 148 registers; above 2048
+// columns the rows' LDS leaves one workgroup of eight waves a CU beside 128, and
+// there the sequence of predictor and correction kernel is the faster one.  us
+// per step, folded (128 registers, 19 spilled) and in sequence: 2049x1024 412
+// and 399, 3001x512 354 and 327, 4096x512 446 and 403, 4096x2048 1677 and 1641,
+// 8192x1024 1711 and 1653; at 2048x1024 342 and 365, at 1100x256 137 and 144.
+bool pred_folds(int itot, int jtot, bool p2) {
+  return p2 || row_shape(itot, jtot).NT <= kFoldDivThreads;
+}
+
 int lu_table_entries(int itot, int jtot) {
   const RowShape r = row_shape(itot, jtot);
   return r.NT * r.M;
@@ -483,7 +493,9 @@ void launch_lu_factor_batch(hipStream_t s, const LuFactorArgs &shape, const LuFa
 
 template <bool P2, bool FOLD, int IMY, class S>
 static void pred_rows_select(hipStream_t s, const PredArgs &shape, S src, int nz) {
-#define SNS_CALL(NT_, M_) pred_rows_launch<NT_, M_, P2, FOLD, IMY>(s, shape, src, nz)
+#define SNS_CALL(NT_, M_)                                       \
+  if constexpr (!FOLD || P2 || NT_ <= kFoldDivThreads) /* pred_folds */ \
+    pred_rows_launch<NT_, M_, P2, FOLD, IMY>(s, shape, src, nz)
   SNS_ROW_DISPATCH(row_shape(shape.g.itot, shape.g.jtot), SNS_CALL);
 #undef SNS_CALL
 }

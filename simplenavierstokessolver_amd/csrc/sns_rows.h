@@ -30,12 +30,13 @@ constexpr int kBlockCols = 124;
 constexpr int kPredGroup = 64;
 
 // Waves per SIMD: the two rows' LDS leaves 4 (two workgroups per CU) at the
-// widest rows; the folded kernel with the division sequence needs 156
-// registers, so on narrower rows it takes 3 (1537x3000: 206 us, 220 with 4 and
-// spilled registers).
-template <bool P2, bool FOLD, int NT>
+// widest rows; the folded kernel with the division sequence needs 148
+// registers, so it takes 3 (1537x3000: 206 us, 220 with 4 and spilled
+// registers), which its widest workgroup, of kFoldDivThreads, still fills.
+constexpr int kFoldDivThreads = 256;
+template <bool P2, bool FOLD>
 constexpr int pred_waves() {
-  return FOLD && !P2 && NT <= 256 ? 3 : 4;
+  return FOLD && !P2 ? 3 : 4;
 }
 
 // Columns of a lane and their byte offsets: in rows of the cell arrays (c,

@@ -251,3 +251,59 @@ def test_state_copies_need_no_state_of_the_instance(sns):
     b.state = None
     a.close()
     b.close()
+
+
+# (itot, jtot, stretch, correction kernels in a step): the widest rows that fold
+# with the division sequence, the first and the widest that do not, and a wide
+# one that divides by multiplying
+FOLD_RULE_CASES = [(2048, 9, 3., 1), (2049, 9, 3., 3), (2049, 1024, 3., 3), (8192, 8, 3., 3),
+                   (4096, 8, 4096., 1), (4097, 8, 4097., 3)]
+
+
+@pytest.mark.parametrize("itot,jtot,stretch,ncorr", FOLD_RULE_CASES)
+def test_fold_rule_of_wide_rows(sns, itot, jtot, stretch, ncorr):
+    """With implicit x the correction is folded into the predictor except where
+    its division sequence would spill registers; the fields are those of the
+    sequence with the correction kernel either way."""
+    out = []
+    for split in (0, 1):
+        inst = sns.Instance(itot, jtot, stretch=stretch, Ra=1e8, Pr=0.7, implicitx=1, implicity=0)
+        inst.set_launch(split_corr=split)
+        inst.state_alloc()
+        rng = np.random.default_rng(itot + jtot)
+        for n in ("ux", "uy", "p", "temp"):
+            inst.state_upload(n, 1e-3 * rng.standard_normal(inst.shape(n)))
+        inst.set_dt(1e-6)
+        inst.timing_enable("corr")
+        inst.integrate()
+        assert inst.timing_read()[0] == (3 if split else ncorr)
+        inst.timing_disable()
+        inst.advance(2)
+        out.append({n: inst.state_download(n) for n in ("ux", "uy", "p", "psi", "temp")})
+        inst.close()
+    for n in out[0]:
+        assert np.array_equal(out[0][n], out[1][n]), n
+
+
+def test_batch_of_wide_rows_mixes_divisors(sns):
+    """A wide uniform member with powers of two for divisors and a stretched
+    one in one class: neither folds, both end where they end alone."""
+    def make(stretch):
+        inst = sns.Instance(4096, 8, stretch=stretch, Ra=1e8, Pr=0.7, implicitx=1, implicity=0)
+        inst.state_alloc()
+        inst.state_init_temperature(3, 1e-2)
+        return inst
+    insts, refs = [make(4096.), make(3.)], [make(4096.), make(3.)]
+    batch = sns.Batch(insts)
+    assert batch.classes() == 1
+    batch.advance(3)
+    for r in refs:
+        r.advance(3)
+    batch.sync()
+    for i, r in zip(insts, refs):
+        for n in ("ux", "uy", "p", "psi", "temp"):
+            assert np.array_equal(i.state_download(n), r.state_download(n)), n
+        assert i.get_time() == r.get_time()
+    batch.close()
+    for i in insts + refs:
+        i.close()
