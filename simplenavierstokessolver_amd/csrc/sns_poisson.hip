@@ -390,9 +390,10 @@ static int one_pass_pairs(int n, int itot) {
   return itot >= 1024 ? 2 : itot >= 256 ? 1 : 0;
 }
 
-// Powers of two have their schedules compiled in, other factors read theirs
-// (registers of the largest radix, a switch per stage: 512x1024 30 us that way,
-// 24 compiled in).
+// Powers of two have their schedules compiled in on either layout, other factors
+// read theirs (registers of the largest radix, a switch per stage: 512x1024 30 us
+// that way, 24 compiled in; passes A and A' on the packed layout, 512x2048 13.3
+// and 6.7 read, 12.4 and 6.3 compiled in).
 using Any = AnySched<16, 3>;
 
 // the two passes' factors
@@ -456,18 +457,18 @@ static void two_pass_sched(const FftSched &sc, F f) {
   else if (FixedSched<8, 16>::is(sc)) f(FixedSched<8, 16>{});
   else f(Any{});
 }
+
 template <class S>
 static void poisson_forward(hipStream_t s, const Fft2Plan &pl, bool pow2, bool aligned, S src,
                             int nz) {
   if (pl.one) return one_pass_forward(s, pl, aligned, src, nz);
   const int T = 1 << pl.lgt, nt = (pl.npair + T - 1) / T;
   const dim3 ga(nt, pl.n2 / pl.G), gb(nt, pl.n1 / 2 + 1);
-  if (!aligned) SNS_FFT_LAUNCH((k_pfwd_a<Any, false, false, S>), pl.G * T, pl.s1, ga);
-  else
-    two_pass_sched(pl.s1, [&](auto sc) {
-      if (pow2) SNS_FFT_LAUNCH((k_pfwd_a<decltype(sc), true, true, S>), pl.G * T, pl.s1, ga);
-      else SNS_FFT_LAUNCH((k_pfwd_a<decltype(sc), false, true, S>), pl.G * T, pl.s1, ga);
-    });
+  two_pass_sched(pl.s1, [&](auto sc) {
+    if (!aligned) SNS_FFT_LAUNCH((k_pfwd_a<decltype(sc), false, false, S>), pl.G * T, pl.s1, ga);
+    else if (pow2) SNS_FFT_LAUNCH((k_pfwd_a<decltype(sc), true, true, S>), pl.G * T, pl.s1, ga);
+    else SNS_FFT_LAUNCH((k_pfwd_a<decltype(sc), false, true, S>), pl.G * T, pl.s1, ga);
+  });
   two_pass_sched(pl.s2, [&](auto sc) {
     SNS_FFT_LAUNCH((k_pfwd_b<decltype(sc), S>), 2 * T, pl.s2, gb);
   });
@@ -481,11 +482,10 @@ static void poisson_inverse(hipStream_t s, const Fft2Plan &pl, bool aligned, S s
   two_pass_sched(pl.s2, [&](auto sc) {
     SNS_FFT_LAUNCH((k_pinv_b<decltype(sc), S>), 2 * T, pl.s2, gb);
   });
-  if (!aligned) SNS_FFT_LAUNCH((k_pinv_a<Any, false, S>), pl.G * T, pl.s1, ga);
-  else
-    two_pass_sched(pl.s1, [&](auto sc) {
-      SNS_FFT_LAUNCH((k_pinv_a<decltype(sc), true, S>), pl.G * T, pl.s1, ga);
-    });
+  two_pass_sched(pl.s1, [&](auto sc) {
+    if (!aligned) SNS_FFT_LAUNCH((k_pinv_a<decltype(sc), false, S>), pl.G * T, pl.s1, ga);
+    else SNS_FFT_LAUNCH((k_pinv_a<decltype(sc), true, S>), pl.G * T, pl.s1, ga);
+  });
 }
 
 template <class S>

@@ -307,3 +307,31 @@ def test_batch_of_wide_rows_mixes_divisors(sns):
     batch.close()
     for i in insts + refs:
         i.close()
+
+
+# (itot, jtot, first factor of the two passes or 0 for the rule, stretch): every
+# pair of compiled schedules (factors of 32, 64 and 128), whole and half tiles
+TWO_PASS_CASES = [(9, 2048, 0, 3.), (16, 2048, 0, 16.), (12, 4096, 0, 3.), (16, 4096, 0, 16.),
+                  (20, 8192, 0, 3.), (8, 8192, 128, 8.), (7, 16384, 0, 3.), (33, 1024, 32, 3.)]
+
+
+@pytest.mark.parametrize("itot,jtot,n1,stretch", TWO_PASS_CASES)
+def test_two_pass_schedules_on_both_layouts(sns, pinned_gauge, itot, jtot, n1, stretch):  # noqa: F811
+    """The two passes with compiled schedules: psi on the packed layout to 1e-11
+    of the oracle's after removing its mean (the bar of the other lengths),
+    and the padded layout's after one fused step equal to it bit for bit."""
+    o, inst = make_pair(sns, itot, jtot, stretch, 0, 0, seed=itot + jtot)
+    inst.set_launch(fft_n1=n1)
+    assert inst.launch()["fft_n1"] >= 32
+    o.compute_potential(1)
+    inst.compute_potential(1)
+    assert_close(interior(inst.download("psi")), interior(o.f["psi"]), 1e-11, "psi", demean=True)
+    inst.state_alloc()
+    for n in ("ux", "uy", "p", "temp"):
+        inst.update_boundaries(n)
+        inst.state_upload(n, inst.download(n))
+    inst.set_dt(1e-8)
+    inst.integrate()
+    inst.integrate_reference_order()
+    assert np.array_equal(inst.state_download("psi"), inst.download("psi"))
+    inst.close()
