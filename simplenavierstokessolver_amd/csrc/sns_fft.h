@@ -299,6 +299,7 @@ struct FixedSched {
     sc.L = 1;
     sc.rmin = r[0];
     for (int p = 0; p < sc.np; p++) {
+      if (r[p] < sc.rmin) sc.rmin = r[p];
       sc.r[p] = r[p];
       sc.ns[p] = FastDiv(sc.L);
       sc.L *= r[p];

@@ -458,6 +458,19 @@ static void two_pass_sched(const FftSched &sc, F f) {
   else f(Any{});
 }
 
+// ... of pass B', with the stages its threads are counted by.  Its first stage
+// reads LDS, so two stages save it nothing, and a last one of radix 16 leaves
+// half of the threads without a butterfly while the others store 16 values each:
+// 4096x8192 147 us with radices 8, 16, 136 with 16, 8, 130 with 8, 4, 4; 8, 8 and
+// 4, 4, 4: 4096x4096 48.7 and 45.4, 2048x4096 26.4 and 23.6, 512x2048 8.4 and 7.2.
+// (More threads beside two stages: 160 us at 4096x8192.)
+template <class F>
+static void pass_b_inverse_sched(const FftSched &sc, F f) {
+  if (FixedSched<8, 8>::is(sc)) f(FixedSched<4, 4, 4>{}, FixedSched<4, 4, 4>::make());
+  else if (FixedSched<8, 16>::is(sc)) f(FixedSched<8, 4, 4>{}, FixedSched<8, 4, 4>::make());
+  else two_pass_sched(sc, [&](auto t) { f(t, sc); });
+}
+
 template <class S>
 static void poisson_forward(hipStream_t s, const Fft2Plan &pl, bool pow2, bool aligned, S src,
                             int nz) {
@@ -479,8 +492,8 @@ static void poisson_inverse(hipStream_t s, const Fft2Plan &pl, bool aligned, S s
   if (pl.one) return one_pass_inverse(s, pl, aligned, src, nz);
   const int T = 1 << pl.lgt, nt = (pl.npair + T - 1) / T;
   const dim3 ga(nt, pl.n2 / pl.G), gb(nt, pl.n1 / 2 + 1);
-  two_pass_sched(pl.s2, [&](auto sc) {
-    SNS_FFT_LAUNCH((k_pinv_b<decltype(sc), S>), 2 * T, pl.s2, gb);
+  pass_b_inverse_sched(pl.s2, [&](auto sc, const FftSched &st) {
+    SNS_FFT_LAUNCH((k_pinv_b<decltype(sc), S>), 2 * T, st, gb);
   });
   two_pass_sched(pl.s1, [&](auto sc) {
     if (!aligned) SNS_FFT_LAUNCH((k_pinv_a<decltype(sc), false, S>), pl.G * T, pl.s1, ga);
