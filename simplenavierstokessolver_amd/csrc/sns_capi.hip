@@ -195,23 +195,13 @@ int ctx_configure(snsg_ctx *c, const snsg_config *cfg, const double *dxf, const 
     t[11][i - 1] = 1. / DXC(i) / DXF(i);
   }
   HIPCHECK(hipMemcpyAsync(c->d_tab, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice, c->stream));
-  // paired copies: (DXC, 1/DXC), (DXF, 1/DXF), (cT_xm, cT_xp), (cU_xm, cU_xp)
-  std::vector<double2> h2(kTables2 * stride);
-  for (size_t k = 0; k < stride; k++) {
-    h2[0 * stride + k] = make_double2(t[1][k], t[3][k]);
-    h2[1 * stride + k] = make_double2(t[0][k], t[2][k]);
-    h2[2 * stride + k] = make_double2(t[4][k], t[5][k]);
-    h2[3 * stride + k] = make_double2(t[6][k], t[7][k]);
-  }
-  HIPCHECK(hipMemcpyAsync(c->d_tab2, h2.data(), sizeof(double2) * h2.size(), hipMemcpyHostToDevice, c->stream));
   Tables &tb = c->tab;
   tb.t = c->d_tab;
-  tb.t2 = c->d_tab2;
   tb.stride = (long)stride;
   tb.dy = dy;
   tb.rdy = 1. / dy;
   // uniform interior: columns I = 2..itot-1 (entry I-1) share every value
-  // the paired tables hold for them; cT_xm(I) for I >= 2 and cT_xp(I) for
+  // the tables of the stencils hold for them; cT_xm(I) for I >= 2 and cT_xp(I) for
   // I <= itot-1 (the same weight), cU_xm and cU_xp likewise
   {
     auto same = [&](const double *v, int from, int to, double &val) {
@@ -346,7 +336,6 @@ extern "C" int snsg_create(int device, const snsg_config *cfg, const double *dxf
       {(void **)&c->d_red, sizeof(unsigned long long)},
       {(void **)&c->d_pack, sizeof(double) * pack_doubles(itot, jtot)},
       {(void **)&c->d_tab, sizeof(double) * kTables * stride},
-      {(void **)&c->d_tab2, sizeof(double2) * kTables2 * stride},
       {(void **)&c->d_pfac, sizeof(double) * nfac},
       {(void **)&c->d_plu, sizeof(double) * 2 * poisson_factor_entries(itot)},
   };
@@ -369,7 +358,7 @@ extern "C" int snsg_destroy(snsg_ctx *c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   void *bufs[] = {c->d_dxf, c->d_dxc, c->d_dt, c->d_eigen, c->d_tw, c->d_psihat, c->d_Y, c->d_q,
                   c->d_qy, c->d_red, c->d_tab, c->d_time, c->d_qf[0], c->d_qf[1],
-                  c->d_qf[2], c->d_lu, c->d_part, c->d_pfac, c->d_tab2, c->d_diag, c->d_plu,
+                  c->d_qf[2], c->d_lu, c->d_part, c->d_pfac, c->d_diag, c->d_plu,
                   c->d_yfac, c->d_qz, c->d_pack};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
@@ -909,7 +898,7 @@ extern "C" int snsg_instance_bytes(const snsg_config *cfg, size_t *bytes) {
   n += z * itot * (jtot / 2 + 1) + z * fft2_work(pl);
   n += 2 * d * (itot + 1) * jtot + sizeof(unsigned long long);
   n += d * pack_doubles((int)itot, (int)jtot);
-  n += d * kTables * stride + z * kTables2 * stride;
+  n += d * kTables * stride;
   n += d * poisson_factor_doubles((int)itot, (int)jtot) + d * 2 * (size_t)poisson_factor_entries((int)itot);
   // snsg_state_alloc
   n += 2 * d * pu * (jtot + 2) + 7 * d * (pc * (jtot + 2) + 16);

@@ -40,7 +40,6 @@ struct snsg_ctx {
   double2 *d_Y = nullptr;  // four-step FFT intermediate, fft2_work entries
   // per-column tables of the fused kernels (one allocation)
   double *d_tab = nullptr;
-  double2 *d_tab2 = nullptr;           // paired column tables
   Tables tab{};
   // fused-step scratch: x-aligned increments of T, ux, uy when a y solve follows
   double *d_qf[3] = {nullptr, nullptr, nullptr};

@@ -71,20 +71,17 @@ __device__ __forceinline__ double from_left(double v) { return dpp_f64<0x138>(v)
 __device__ __forceinline__ double from_right(double v) { return dpp_f64<0x130>(v); }
 // Per-column tables, all indexed like the reference arrays they derive from
 // (entry I-1 holds the value for column I unless noted).  They live in one
-// allocation of 14 double tables and one of 4 double2 tables, each table
-// `stride` entries long, so an instance's tables cost two pointers.
-// number of double and of double2 tables
-constexpr int kTables = 14, kTables2 = 4;
+// allocation of kTables tables, each `stride` entries long.
+constexpr int kTables = 14;
 
 struct Tables {
   const double *t;             // 14 tables, in the order of the accessors below
-  const double2 *t2;           // 4 paired tables
   long stride;
   double dy, rdy;
   // Set when the grid is uniform bit for bit away from the walls: every
   // column I = 2..itot-1 has the same DXF, DXC and interpolation weights
   // (u_*).  A wave whose columns all lie there uses these values instead of
-  // loading the paired tables; the values are the table entries themselves.
+  // loading the tables; the values are the table entries themselves.
   int uniform;
   double u_dxc, u_rdxc, u_dxf, u_rdxf, u_cT, u_cU;
   // Set when every divisor of the stencils (DXF, DXC of all columns and dy)
@@ -117,11 +114,6 @@ struct Tables {
   // 1./DXC(I)/DXF(I), 1./DXC(I+1)/DXF(I)       (Poisson)
   __host__ __device__ const double *pl() const { return tab(12); }
   __host__ __device__ const double *pu() const { return tab(13); }
-  // the same values in pairs, for one 16-byte load each (entry as above)
-  __host__ __device__ const double2 *dxc2() const { return t2; }               // (DXC, 1./DXC)
-  __host__ __device__ const double2 *dxf2() const { return t2 + stride; }      // (DXF, 1./DXF)
-  __host__ __device__ const double2 *cT2() const { return t2 + 2 * stride; }   // (cT_xm, cT_xp)
-  __host__ __device__ const double2 *cU2() const { return t2 + 3 * stride; }   // (cU_xm, cU_xp)
 };
 
 // Host: whether the kernels take the power-of-two division path for these
@@ -183,9 +175,9 @@ struct Weights {
 // Temperature at (i, j) and its neighbours, with the velocities it is
 // advected by: src/temperature/update.c:33-84
 struct TempPt {
-  double t_c, t_xm, t_xp, t_ym, t_yp;  // T(i,j), T(i-1,j), T(i+1,j), T(i,j-1), T(i,j+1)
-  double ux_c, ux_p;                   // UX(i,j), UX(i+1,j)
-  double uy_c, uy_p;                   // UY(i,j), UY(i,j+1)
+  double t_c, t_ym, t_yp;  // T(i,j), T(i,j-1), T(i,j+1)
+  double ux_c, ux_p;       // UX(i,j), UX(i+1,j)
+  double uy_c, uy_p;       // UY(i,j), UY(i,j+1)
 };
 // Column metrics of cell i: DXC(i), DXC(i+1), DXF(i) with reciprocals and the
 // interpolation weights DXC(i)/(2DXF(i)), DXC(i+1)/(2DXF(i))
@@ -193,9 +185,8 @@ struct CellX {
   double dxc, rdxc, dxc_p, rdxc_p, dxf, rdxf, c_xm, c_xp;
 };
 // The x-gradients at the faces of cell i, dtdx_xm = (T(i)-T(i-1))/DXC(i) and
-// dtdx_xp = (T(i+1)-T(i))/DXC(i+1), are given (the t_xm, t_xp entries of v
-// are not read): a kernel holding consecutive columns forms each face
-// gradient once and hands it to both cells.
+// dtdx_xp = (T(i+1)-T(i))/DXC(i+1), are given: a kernel holding consecutive
+// columns forms each face gradient once and hands it to both cells.
 template <bool P2 = false, class W>
 __device__ __forceinline__ void temp_src_g(const Geo &g, const Tables &tb, const CellX &x,
                                            const TempPt &v, double dtdx_xm, double dtdx_xp,
@@ -218,13 +209,13 @@ struct UxPt {
   double p_c, p_m;                     // P(i,j), P(i-1,j)
   double tf;                           // buoyancy at the face
 };
-// Face metrics of face i: DXF(i-1), DXF(i) with reciprocals, the weights
-// DXF(i-1)/(2DXC(i)), DXF(i)/(2DXC(i)) and DXC(i) with its reciprocal
+// Metrics of face i: the weights DXF(i-1)/(2DXC(i)), DXF(i)/(2DXC(i)) and
+// DXC(i) with its reciprocal
 struct FaceX {
-  double dxf_m, rdxf_m, dxf, rdxf, c_xm, c_xp, dxc, rdxc;
+  double c_xm, c_xp, dxc, rdxc;
 };
 // The x-gradients (UX(i)-UX(i-1))/DXF(i-1) and (UX(i+1)-UX(i))/DXF(i) are
-// given, as for temp_src_g (u_xm and u_xp still enter the interpolations).
+// given, as for temp_src_g (u_xm and u_xp enter the interpolations).
 template <bool P2 = false, class W>
 __device__ __forceinline__ void ux_src_g(const Geo &g, const Tables &tb, const FaceX &x,
                                          const UxPt &v, double duxdx_xm, double duxdx_xp,
@@ -247,9 +238,9 @@ __device__ __forceinline__ void ux_src_g(const Geo &g, const Tables &tb, const F
 
 // y-momentum at (i, j), i = 1..itot: src/fluid/update_velocity.c:128-189
 struct UyPt {
-  double v_c, v_xm, v_xp, v_ym, v_yp;  // UY(i,j), UY(i-1,j), UY(i+1,j), UY(i,j-1), UY(i,j+1)
-  double ux_mc, ux_cc, ux_mp, ux_cp;   // UX(i,j-1), UX(i,j), UX(i+1,j-1), UX(i+1,j)
-  double p_c, p_ym;                    // P(i,j), P(i,j-1)
+  double v_c, v_ym, v_yp;             // UY(i,j), UY(i,j-1), UY(i,j+1)
+  double ux_mc, ux_cc, ux_mp, ux_cp;  // UX(i,j-1), UX(i,j), UX(i+1,j-1), UX(i+1,j)
+  double p_c, p_ym;                   // P(i,j), P(i,j-1)
 };
 // The x-gradients (UY(i)-UY(i-1))/DXC(i) and (UY(i+1)-UY(i))/DXC(i+1) are
 // given, as for temp_src_g.

@@ -402,8 +402,8 @@ __device__ __forceinline__ void raw_eval(const PredArgs &a, const Q &q, const Ra
   double2 A, G;
   if constexpr (F == 1) {
     // faces: metrics DXC(i) and the weights; gradients over cells
-    const FaceX x0 = {0., 0., m.dxf.x, m.rdxf.x, m.wm.x, m.wp.x, m.dxc.x, m.rdxc.x};
-    const FaceX x1 = {0., 0., m.dxf.y, m.rdxf.y, m.wm.y, m.wp.y, m.dxc.y, m.rdxc.y};
+    const FaceX x0 = {m.wm.x, m.wp.x, m.dxc.x, m.rdxc.x};
+    const FaceX x1 = {m.wm.y, m.wp.y, m.dxc.y, m.rdxc.y};
     auto row = [&](double2 u_s, double2 u, double2 u_n, double2 v_s,
                    double2 v_n, double vl_s, double vl_n, double2 pc,
                    double2 t) {
@@ -436,8 +436,8 @@ __device__ __forceinline__ void raw_eval(const PredArgs &a, const Q &q, const Ra
         const double g0 = dv<P2>(-t.x + t.y, m.dxc.y, m.rdxc.y);
         const double g1 = dv<P2>(-t.y + tr, dxc_r, rdxc_r);
         const double gl = from_left(g1);
-        const TempPt p0 = {t.x, 0., 0., t_s.x, t_n.x, u.x, u.y, v_s.x, v_n.x};
-        const TempPt p1 = {t.y, 0., 0., t_s.y, t_n.y, u.y, ur, v_s.y, v_n.y};
+        const TempPt p0 = {t.x, t_s.x, t_n.x, u.x, u.y, v_s.x, v_n.x};
+        const TempPt p1 = {t.y, t_s.y, t_n.y, u.y, ur, v_s.y, v_n.y};
         temp_src_g<P2>(g, tb, x0, p0, gl, g0, w, A.x, G.x);
         temp_src_g<P2>(g, tb, x1, p1, g0, g1, w, A.y, G.y);
       };
@@ -451,8 +451,8 @@ __device__ __forceinline__ void raw_eval(const PredArgs &a, const Q &q, const Ra
         const double g0 = dv<P2>(-v.x + v.y, m.dxc.y, m.rdxc.y);
         const double g1 = dv<P2>(-v.y + vr, dxc_r, rdxc_r);
         const double gl = from_left(g1);
-        const UyPt p0 = {v.x, 0., 0., v_s.x, v_n.x, u_s.x, u.x, u_s.y, u.y, pc.x, p_s.x};
-        const UyPt p1 = {v.y, 0., 0., v_s.y, v_n.y, u_s.y, u.y, ur_s, ur, pc.y, p_s.y};
+        const UyPt p0 = {v.x, v_s.x, v_n.x, u_s.x, u.x, u_s.y, u.y, pc.x, p_s.x};
+        const UyPt p1 = {v.y, v_s.y, v_n.y, u_s.y, u.y, ur_s, ur, pc.y, p_s.y};
         uy_src_g<P2>(g, tb, x0, p0, gl, g0, w, A.x, G.x);
         uy_src_g<P2>(g, tb, x1, p1, g0, g1, w, A.y, G.y);
       };
