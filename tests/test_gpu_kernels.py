@@ -110,7 +110,7 @@ def test_row_predictor_edges(sns, itot, jtot, imy):
 
 
 # itot at the edges of the blocks (124 columns) and of the workgroups (four
-# blocks), odd row counts; powers of two with stretch 0 divide by multiplying
+# blocks), odd row counts; stretch 0 is the Chebyshev grid
 EXP_CASES = [(4, 4, 0.), (5, 9, 3.), (64, 64, 0.), (123, 12, 3.), (124, 15, 0.), (125, 12, 3.),
              (128, 192, 0.), (248, 9, 3.), (249, 8, 0.), (497, 12, 3.), (512, 32, 0.),
              (1024, 15, 0.)]
@@ -335,3 +335,49 @@ def test_two_pass_schedules_on_both_layouts(sns, pinned_gauge, itot, jtot, n1, s
     inst.integrate_reference_order()
     assert np.array_equal(inst.state_download("psi"), inst.download("psi"))
     inst.close()
+
+
+# Uniform grids: powers of two for every divisor (the kernels multiply), uniform
+# spacings in x with another dy (they divide, with the spacings of interior
+# blocks as constants), and widths whose uniform spacings differ in their last
+# bits (they divide by the tables'); one block to many, one to several workgroups
+# per row
+UNIFORM_CASES = [(4, 4, True), (64, 64, True), (128, 16, True), (256, 8, True), (512, 32, True),
+                 (512, 2048, True), (1024, 16, True), (2048, 8, True), (4096, 8, True),
+                 (8192, 4, True), (128, 15, False), (256, 90, False), (512, 45, False),
+                 (1024, 1080, False), (2048, 12, False), (4096, 9, False), (250, 8, False),
+                 (373, 12, False), (500, 15, False), (1000, 16, False), (3000, 9, False)]
+
+
+@pytest.mark.parametrize("imx,imy", [(0, 0), (1, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("itot,jtot,pow2", UNIFORM_CASES)
+def test_predictors_on_uniform_grids(sns, itot, jtot, pow2, imx, imy):
+    """Two fused steps against the reference-named functions, whose source
+    terms equal the oracle's bit for bit: every field equal."""
+    if imy and jtot < 16:
+        jtot = 16 if pow2 else 18
+    fields = {}
+    for fused in (False, True):
+        inst = sns.Instance(itot, jtot, stretch=float(itot), Ra=1e7, Pr=2.0, implicitx=imx,
+                            implicity=imy)
+        assert inst.uniform_grid() == (itot & (itot - 1) == 0)
+        spacings = list(inst.g["dxf"]) + list(inst.g["dxc"]) + [2.0 / jtot]
+        assert all(np.frexp(v)[0] == 0.5 for v in spacings) == pow2
+        inst.alloc()
+        inst.state_alloc()
+        rng = np.random.default_rng(itot + jtot)
+        for n in ("ux", "uy", "p", "temp"):
+            inst.upload(n, 0.1 * rng.standard_normal(inst.shape(n)))
+            inst.update_boundaries(n)
+            inst.state_upload(n, inst.download(n))
+        inst.set_dt(1e-7)
+        for _ in range(2):
+            inst.integrate() if fused else inst.integrate_reference_order()
+        for n in ("ux", "uy", "p", "temp"):
+            inst.update_boundaries(n)
+            got = inst.state_download(n) if fused else inst.download(n)
+            assert np.isfinite(got).all()
+            if fused:
+                assert np.array_equal(got, fields[n]), (n, np.abs(got - fields[n]).max())
+            fields[n] = got
+        inst.close()
