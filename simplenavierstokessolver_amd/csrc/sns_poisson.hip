@@ -468,7 +468,8 @@ template <class F>
 static void pass_b_inverse_sched(const FftSched &sc, F f) {
   if (FixedSched<8, 8>::is(sc)) f(FixedSched<4, 4, 4>{}, FixedSched<4, 4, 4>::make());
   else if (FixedSched<8, 16>::is(sc)) f(FixedSched<8, 4, 4>{}, FixedSched<8, 4, 4>::make());
-  else two_pass_sched(sc, [&](auto t) { f(t, sc); });
+  else if (FixedSched<4, 8>::is(sc)) f(FixedSched<4, 8>{}, sc);
+  else f(Any{}, sc);
 }
 
 template <class S>
