@@ -227,8 +227,8 @@ typedef struct {
                            increments) */
   int ysolve_cols;      /* columns per workgroup of its interface solve: 16,
                            32 or 64 (set, it keeps the solve in three
-                           kernels; the rule takes one kernel up to 256
-                           chunks) */
+                           kernels; the rule takes one kernel up to 128
+                           chunks, 256 up to 1024 columns) */
   int ysolve_recompute; /* its chunk interiors: 1 solved again in the apply
                            kernel, 2 stored and read back */
   int split_corr;       /* 1: every substage ends with the correction kernel;

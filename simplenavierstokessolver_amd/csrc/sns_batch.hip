@@ -7,7 +7,8 @@
 // member's argument blocks in a device table (ArgBatch), on the lane's own
 // stream; the lane's step is recorded once as a HIP graph and replayed.  The
 // kernels are the single-instance ones, so every member advances bitwise as
-// it would alone.
+// it would alone (whether they divide by multiplying is the members' common
+// choice: lane_build).
 #include <math.h>
 #include <string.h>
 
@@ -429,7 +430,8 @@ struct Pooled {
 // step.  A second step is enqueued behind the running one, so the device does
 // not wait for the engine between them (four jobs of 128x256 to 512x1024, 100 to
 // 150 steps: 113 ms with their downloads, 118 with one step at a time), unless the
-// membership changes there: a job joined, or one of the running step's ends.
+// membership changes there: a job joined, or one of the running step's ends.  A job
+// that joins waits for the steps in flight, two at most.
 constexpr int kAhead = 2;
 struct ServeLane {
   Lane k;

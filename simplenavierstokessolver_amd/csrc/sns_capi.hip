@@ -1272,8 +1272,9 @@ void step_args(const snsg_ctx *c, const snsg_state *st, bool reduce, bool p2, St
       if (pa.p_out) in_p = pa.p_out;
     }
   }
-  // The first kernel decides dt where that is cheap: 18 workgroups of factors
-  // read up to 2048 partials each, the predictor's, in their hundreds, 512.
+  // The first kernel decides dt where that is cheap: every wave of the nine
+  // workgroups of factors reads up to 2048 partials, every wave of the predictor's,
+  // in their hundreds, 512.
   const bool yfac = impy && sa.yf.L;
   sa.dt_first = reduce && c->nparts <= (impx || yfac ? 2048 : 512);
   if (sa.dt_first) (impx ? sa.lu.dt : yfac ? sa.yf.dt : sa.pred[0].dt) = sa.dt;

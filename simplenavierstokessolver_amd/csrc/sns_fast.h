@@ -145,8 +145,8 @@ __device__ __forceinline__ void str(double *row, int k, double v) {
 // ------------------------------------------------------------ source terms
 //
 // Each source term is written once, on the values around the point; the
-// predictors feed it with values shared across lanes and rows (sns_rows.h).  Operation order follows the reference
-// expression by expression.
+// predictors feed it with values shared across lanes and rows (sns_rows.h).
+// Operation order follows the reference expression by expression.
 
 // Split of the diffusive terms dif1 (x), dif2 (y) between the explicit part
 // A and the implicit part G.  IX, IY: the treatment of x and y where the

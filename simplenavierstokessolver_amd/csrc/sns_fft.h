@@ -3,11 +3,15 @@
 // Stockham auto-sort stages (no bit reversal): the stage with radix R and
 // running sub-transform length Ns reads x_r = buf[j + r*L/R], applies the
 // twiddles w^(r*k), k = j mod Ns, w = exp(sign*2*pi*i/(Ns*R)), performs an
-// R-point DFT and writes buf[(j-k)*R + k + r*Ns].  A transform takes two
-// stages (three where its length has no two factors up to 16), one butterfly
-// per thread and stage: the first stage's inputs and the last one's outputs
-// pass through registers only, so a transform costs one LDS exchange and one
-// barrier where staging every stage in LDS cost four and six.
+// R-point DFT and writes buf[(j-k)*R + k + r*Ns].  One butterfly per thread and
+// stage.  The first stage may take its inputs in registers and the last one
+// leave its outputs there: two stages between global memory and global memory
+// (passes A and A' of the two-pass transforms, lengths with two factors up to 16)
+// cost one LDS exchange and one barrier where staging each in LDS cost four and
+// six.  Every further stage is an exchange more, with two barriers: three stages
+// where a length has no two such factors, three or four in the transforms of
+// whole columns, whose radices are kept small; and the side of a transform where
+// spectra are separated or combined goes through LDS.
 //
 // Twiddles come from a table tw[m] = exp(-2*pi*i*m/n) evaluated on the host
 // (those of the length L in LDS); the inverse transform uses their

@@ -1,14 +1,19 @@
 // sns_fused.hip -- fused substage kernels for the time-step hot path (gfx950).
 //
-// One RK substage (src/main.c:81-98) becomes five kernels:
+// One RK substage (src/main.c:81-98) becomes these kernels:
 //   pred : T, ux and uy predictors in one pass over the substage-start fields
-//          (buoyancy from T in registers, RK history read/written in place,
-//          Crank-Nicolson in x solved on chip for a whole row), writing
-//          T' (ping-pong buffer), ux*, uy* with their boundary values;
-//   poisson_fwd / poisson_x / poisson_inv : the potential (sns_solve.hip);
+//          (buoyancy from T in registers, RK history read/written in place),
+//          writing T' (ping-pong buffer), ux*, uy* with their boundary values:
+//          explicit x here, with Crank-Nicolson in x solved on chip for a
+//          whole row in sns_pred.hip; the increments alone where y is implicit,
+//          whose solve follows (sns_ysolve.hip);
+//   poisson_fwd / poisson_x / poisson_inv : the potential (sns_poisson.hip, the
+//          transforms up to 1024 rows in sns_poisson_one.hip);
 //   corr : velocity correction and pressure update in one pass, plus on
 //          the last substage the advective time-step bound for the next
-//          step (a min-reduction over the corrected velocities).
+//          step (a min-reduction over the corrected velocities).  With
+//          explicit y the predictors of substages 2 and 3 apply the one of
+//          substages 1 and 2 instead (step_args).
 // The explicit and implicit diffusive parts, the RK increments and the
 // boundary values follow the reference expression for expression (see
 // sns_fast.h for the division scheme); only the line solves round

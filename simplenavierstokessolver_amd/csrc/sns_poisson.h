@@ -24,7 +24,7 @@ struct Fft2Plan {
 // first factor (false when the factors or the LDS tiles do not fit)
 bool fft2_plan(int n, int itot, Fft2Plan &pl, int n1 = 0);
 
-// Entries of the two passes' intermediate (whole tiles of 8 pairs)
+// Entries of the two passes' intermediate (pairs rounded up to 16, whole tiles of 8)
 inline size_t fft2_work(const Fft2Plan &pl) { return (size_t)(pl.npair + 15) / 16 * 16 * pl.n; }
 
 // Thomas factors of the x systems of all wavenumbers (once per instance):

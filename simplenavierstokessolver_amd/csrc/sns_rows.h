@@ -194,9 +194,9 @@ __device__ __forceinline__ double2 hist_load(Buf h, const LanePos &p, unsigned r
   return v;
 }
 
-// The rows are loaded and evaluated one after the other (PART 0: what row ja
-// needs, 1: what row jb needs besides), which keeps a third fewer values in
-// registers than loading both first.
+// PART 0: what row ja needs, 1: what row jb needs besides.  k_pred_rows loads and
+// evaluates the rows one after the other, which keeps a third fewer values in
+// registers than loading both first; k_pred_exp, bound by latency, loads both.
 template <int F, bool P2, bool FOLD, int PART>
 __device__ __forceinline__ void raw_load(const Tables &tb, const RowSrc<F, FOLD> &q,
                                          const LanePos &p, Raw<F> &r) {

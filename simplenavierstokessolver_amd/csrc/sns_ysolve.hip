@@ -19,7 +19,8 @@
 //     (src/linalg.c:52-108): the (S-1)-row block with the right-hand side
 //     and with [-O, 0, .., 0, -O], then the last unknown, then the rest.
 // k_ycol does all of it in one kernel, a workgroup holding whole columns (the
-// rule's choice up to 256 chunks).  Otherwise, three kernels: k_ylocal
+// rule's choice up to 128 chunks, 256 on narrow grids: ysolve_one_pass).
+// Otherwise, three kernels: k_ylocal
 // (the interior solves; the first and last interior
 // values of each chunk go to qz rows S..3S-1), k_yreduced (the interface
 // system, one wave per column, into qz rows 0..S-1), k_yapply (the
@@ -30,8 +31,8 @@
 // interior solution and k_yapply_rows applies it row by row (one thread per
 // cell, which keeps small instances busy).  The factors of T and of the
 // reduced system depend on dt; k_yfactor computes them once per step for the
-// three substages and fields.  Rounding differs from the reference's sequential sweep at the
-// ulp level.
+// three substages and fields.  Rounding differs from the reference's sequential
+// sweep at the ulp level.
 #include "sns_launch.h"
 #include "sns_fast.h"
 #include "sns_fused.h"
