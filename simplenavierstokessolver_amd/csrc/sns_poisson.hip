@@ -16,12 +16,12 @@
 // separated (forward) or combined (inverse) in pass B / B', which therefore
 // handles the wavenumber rows k1 and n1-k1 together.
 //
-// The passes move 3, 2, 2 and 2 words per cell; from 4096x8192 (4.1, 4.8, 3.8
+// The passes move 3, 2, 2 and 2 words per cell; from 4096x8192 (4.1, 5.0, 4.4
 // and 4.6 TB/s) they are bound by memory, whose rate the short strided runs
 // keep under that of a copy; smaller grids by a workgroup's chain of latencies.
 // us of the four passes with every stage through LDS, and with the first and
-// last stage in registers and Y in one run per tile: 1537x3000 129 and 108,
-// 1024x2048 50 and 44, 2048x4096 143 and 134, 4096x8192 570 and 562.
+// last stage in registers and Y in one run per tile: 1537x3000 130 and 109,
+// 1024x2048 50 and 44, 2048x4096 138 and 133, 4096x8192 571 and 543.
 #include <float.h>
 #include "sns_launch.h"
 #include "sns_fast.h"

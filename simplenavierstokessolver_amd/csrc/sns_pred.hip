@@ -14,11 +14,12 @@
 // does not start on a cache line costs a line more.  Evaluating one block of
 // a wave's own contiguous columns after the other, so that the lines at the
 // block ends were fetched twice, took 0.96 ms where the waves of a workgroup
-// side by side take 0.80; loads issued a block ahead did not help.  With one
+// side by side take 0.85; loads issued a block ahead did not help.  With one
 // column per lane and unrolled blocks (15900 instructions, 1700 of them moving
 // spilled scalars) it took 0.93.  us per launch, before and now: 4096x8192
-// 925 and 800, folded 1285 and 1067; 2048x4096 244 and 189; 1537x3000 163 and
-// 143; 512x1024 24.4 and 18.1; 225x360 13.8 and 9.8, folded 16.9 and 11.4.
+// 929 and 865, folded 1288 and 1134; 2048x4096 244 and 202; 1537x3000 164 and
+// 146, folded 221 and 203; 512x1024 24.1 and 18.5; 225x360 13.9 and 9.0, folded
+// 16.9 and 11.4.
 #include "sns_launch.h"
 #include "sns_fast.h"
 #include "sns_fused.h"
